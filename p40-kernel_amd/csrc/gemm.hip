@@ -1288,6 +1288,8 @@ int64_t gemm_wide_rows(const void * W, const void * Xq, int64_t n_out, int64_t n
 int gemm_wide_launch(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
                      hipStream_t st);
 int64_t gemm_wide_x16_bytes(int64_t n_tok, int nb);
+// gemm_mid.hip: small tiles with K split over a workgroup's waves; -1 if not applicable
+int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st);
 int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
                         void * ws, hipStream_t st);
 }
@@ -1372,6 +1374,13 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
                 return gemm_prefill_f16(w + (size_t)rows * PQ2_BYTES * nb, x, Y + (size_t)rows * n_tok,
                                         n_out - rows, n_tok, nb, st);
             }
+        }
+        // what the wide kernel leaves: small tiles where 128-row tiles would
+        // leave most CUs idle (BONSAI_GEMM_WIDE other than 1 compares the tile
+        // kernels, which add in one order)
+        if (wide == 1 || knob(pq2host::K_GEMM_MID, -1) > 0) {
+            const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, gemm_cu_count(), st);
+            if (rc >= 0) return rc;
         }
         return gemm_prefill_f16(w, x, Y, n_out, n_tok, nb, st);
     } else if ((nb & 1) || ((uintptr_t)W & 3u) != 0) {
