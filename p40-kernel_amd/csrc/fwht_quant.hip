@@ -92,16 +92,22 @@ quant_kernel(const float * __restrict__ x, uint8_t * __restrict__ q, int nchunk,
 }
 
 // RMSNorm -> FWHT -> Q8_1 of token rows (src/ops.h:13-22, then the pre-pass
-// above).  Grid n_tok, one workgroup per token, nw = min(n / 1024, 16) waves;
-// wave w owns the Hadamard blocks w, w + nw, ...  The sum of squares is
-// accumulated in fp64 in the one order every normalising kernel uses
-// (rms_sumsq: per-block lane sums, a wave tree, blocks in order), so every
+// above), many tokens.  Grid n_tok, one workgroup per token, nw waves; wave w
+// owns the Hadamard blocks w, w + nw, ... (KEEP of them held in registers from
+// the sum of squares to the quantiser; KEEP = 0: read again).  The sum of
+// squares is accumulated in fp64 in the one order every normalising kernel
+// uses (rms_sumsq: per-block lane sums, a wave tree, blocks in order), so every
 // path computes the same s = 1 / sqrtf((float)(ss / n) + eps); the
 // reference's sequential fp32 sum differs from it by that sum's own rounding.
 // Then y = (x * s) * w, the signs, the register FWHT and the quantiser, as
-// the pre-pass.  Output
-// chunk-major (block (c, t) at c * n_tok + t; for one token the GEMV layout).
-template <bool VEC, bool SIGNS>
+// the pre-pass.  Output chunk-major (block (c, t) at c * n_tok + t).
+// Workgroups go to the 8 XCDs in turn: each XCD takes a contiguous run of
+// tokens, whose 36-byte blocks share lines of its L2.  VALU-bound (~600
+// instructions a block) at about the time its bytes take: with the row read
+// once and the tokens dealt by XCD 2048 x 5120 went 20.1 -> 17.0 us (54 MB,
+// 3.2 TB/s), 2048 x 17408 67.6 -> 52.6.  Collecting 2 or 4 tokens a workgroup
+// to write longer runs measured slower (18.5, 22.1).
+template <bool VEC, bool SIGNS, int KEEP>
 __global__ void __launch_bounds__(1024)
 rms_rot_quant_kernel(const float * __restrict__ x, const float * __restrict__ w,
                      const float * __restrict__ signs, uint8_t * __restrict__ q, int n, int n_tok,
@@ -109,19 +115,33 @@ rms_rot_quant_kernel(const float * __restrict__ x, const float * __restrict__ w,
     __shared__ double red[RMS_GROUP];
     const int l = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const int tok = blockIdx.x;
+    const int xcd = blockIdx.x & 7;
+    const int tok = xcd * (n_tok >> 3) + min(xcd, n_tok & 7) + ((int)blockIdx.x >> 3);
     const int nhb = n / HBLK;
     const int row = fwht_row(l);
     const float * xt = x + (size_t)tok * n;
 
-    const double tot = rms_sumsq(
-        nhb, red, nw, wave, l, [&](int b, float (&v)[16]) { load16(xt + (size_t)HBLK * b + 16 * row, v, VEC); },
-        [] { __syncthreads(); });
+    float held[KEEP ? KEEP : 1][16];
+    if constexpr (KEEP > 0) {
+#pragma unroll
+        for (int k = 0; k < KEEP; ++k)
+            if (wave + k * nw < nhb) load16(xt + (size_t)HBLK * (wave + k * nw) + 16 * row, held[k], VEC);
+    }
+    // (a wave's blocks come in the order k = 0, 1, ...)
+    auto block = [&](int b, float (&v)[16]) {
+        if constexpr (KEEP == 0) {
+            load16(xt + (size_t)HBLK * b + 16 * row, v, VEC);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = KEEP == 2 && b >= nw ? held[KEEP - 1][r] : held[0][r];
+        }
+    };
+    const double tot = rms_sumsq(nhb, red, nw, wave, l, block, [] { __syncthreads(); });
     const float s = 1.0f / sqrtf((float)(tot / (double)n) + eps);
 
     for (int b = wave; b < nhb; b += nw) {
         float v[16], wv[16];
-        load16(xt + (size_t)HBLK * b + 16 * row, v, VEC);
+        block(b, v);
         load16(w + (size_t)HBLK * b + 16 * row, wv, VEC);
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = v[r] * s * wv[r];
@@ -304,18 +324,28 @@ int bonsai_p40_rmsnorm_fwht_quant(const float * x, const float * w, const float 
     if (n <= 0 || n % HBLK != 0 || pq2host::any_null(x, w, xq) || !al4(xq)) return 1;
     if (n_tok <= 0) return 0;
     if (n_tok > 0x7fffffff || n > 0x7fffffff) return 1;
-    const int nw = (int)(n / HBLK < 16 ? n / HBLK : 16);
+    // one block a wave where they fit, two where that is enough (17 blocks: 9 waves)
+    const int nhb = (int)(n / HBLK), keep = nhb <= 16 ? 1 : nhb <= 32 ? 2 : 0;
+    const int nw = keep == 1 ? nhb : keep == 2 ? (nhb + 1) / 2 : 16;
     const bool vec = al16(x) && al16(w) && al16(signs);
     hipStream_t st = (hipStream_t)stream;
     // few tokens: a workgroup per block (spread over the CUs); many: one per
-    // token (each token row read once)
-    const bool per_block = n_tok * (n / HBLK) <= 4096 && n_tok <= 65535 && n / HBLK <= 0x7fffffff;
+    // token (each token row read once).  Measured on MI355X (us, per block /
+    // per token): 32 x 5120 4.0 / 4.6, 64 x 5120 4.5 / 4.5, 130 x 5120 5.8 /
+    // 4.6, 512 x 5120 12.1 / 6.7, 40 x 17408 7.9 / 7.3, 100 x 17408 13.0 / 7.6
+    const bool per_block = n_tok * (n / HBLK) <= 256;
 #define PQ2_RMS_LAUNCH(V, S)                                                                        \
     if (per_block)                                                                                  \
         hipLaunchKernelGGL((rms_rot_quant_block_kernel<V, S>), dim3((unsigned)(n / HBLK), (unsigned)n_tok), \
                            dim3(256), 0, st, x, w, signs, (uint8_t *)xq, (int)n, (int)n_tok, eps);  \
+    else if (keep == 1)                                                                             \
+        hipLaunchKernelGGL((rms_rot_quant_kernel<V, S, 1>), dim3((unsigned)n_tok), dim3(64 * nw), 0, st, \
+                           x, w, signs, (uint8_t *)xq, (int)n, (int)n_tok, eps);                    \
+    else if (keep == 2)                                                                             \
+        hipLaunchKernelGGL((rms_rot_quant_kernel<V, S, 2>), dim3((unsigned)n_tok), dim3(64 * nw), 0, st, \
+                           x, w, signs, (uint8_t *)xq, (int)n, (int)n_tok, eps);                    \
     else                                                                                            \
-        hipLaunchKernelGGL((rms_rot_quant_kernel<V, S>), dim3((unsigned)n_tok), dim3(64 * nw), 0, st, \
+        hipLaunchKernelGGL((rms_rot_quant_kernel<V, S, 0>), dim3((unsigned)n_tok), dim3(64 * nw), 0, st, \
                            x, w, signs, (uint8_t *)xq, (int)n, (int)n_tok, eps)
     if (vec && signs) PQ2_RMS_LAUNCH(true, true);
     else if (vec) PQ2_RMS_LAUNCH(true, false);

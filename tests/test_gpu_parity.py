@@ -1223,3 +1223,22 @@ def test_unit_dma_probe_runs(n_out, n_in):
         B.unit_dma_probe(W, n_out, n_in, sink)
     torch.cuda.synchronize()
     assert int(sink.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("n,n_tok", [(1024, 257), (5120, 51), (5120, 52), (16384, 17), (17408, 16), (17408, 301),
+                                     (32768, 9), (33792, 9)])
+def test_rms_prepass_tokens_equal_single_rows(n, n_tok):
+    """The many-token kernel (one block, two blocks or more per wave, token
+    counts that do not divide by 8, either side of the choice between the two
+    kernels): the bytes of one call per token."""
+    case(f"rmsnorm_fwht_quant {n_tok} x {n} against single rows")
+    x = dev(O.gen_normal(2900 + n, n * n_tok))
+    w, signs = dev(O.gen_normal(2901, n) * 0.1 + 1), dev(np.where(O.gen_normal(2902, n) < 0, -1, 1).astype(np.float32))
+    got = torch.zeros(B.q8_bytes(n, n_tok), dtype=torch.uint8, device="cuda")
+    B.rmsnorm_fwht_quant(x, w, signs, got, n, n_tok, 1e-6)
+    rows = []
+    for t in range(n_tok):
+        row = torch.zeros(B.q8_bytes(n), dtype=torch.uint8, device="cuda")
+        B.rmsnorm_fwht_quant(x[t * n:(t + 1) * n], w, signs, row, n, 1, 1e-6)
+        rows.append(host(row).reshape(-1, 36))
+    np.testing.assert_array_equal(host(got).reshape(n // 32, n_tok, 36), np.stack(rows, axis=1))
