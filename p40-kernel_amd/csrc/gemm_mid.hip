@@ -212,6 +212,7 @@ gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, 
                 for (int ni = 0; ni < NI; ++ni) {
                     Bf[ni] = q_f16(xw[ni][1], xw[ni][2]);
                     da[c & 1][ni] = f16_bits_to_f32(xw[ni][0] & 0xffffu);
+                    asm("" : "+v"(da[c & 1][ni]));              // fp32 from here on, not an f16 source of each FMA
                     E[ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fix, Bf[ni], (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
                 }
             }
