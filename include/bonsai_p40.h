@@ -64,7 +64,8 @@ int bonsai_p40_quant_activations(const float * x, void * out, int64_t n, bonsai_
 // per-token activation planes; 3..8 the block-diagonal 16x16x64 int8 MFMA
 // kernel, except 4 tokens on 1024-, 5120- and 6144-column rows and 3 on
 // 1024- and 6144-column rows, which take the 4x4x4 int8 MFMA streaming
-// kernel; 9..16 the streamed 16x16x32 int8 MFMA kernel; larger n_tok the
+// kernel; 9..16 the streamed 16x16x32 int8 MFMA kernel, or on tall matrices
+// (17408 rows) f16-MFMA 80x16 tiles that read s as it does; larger n_tok the
 // f16-MFMA tile GEMMs: small tiles with K split over a workgroup's waves
 // where larger ones would leave CUs idle (n_in % 1024 == 0, 16-byte aligned
 // W), else 128- to 256-row tiles (other alignments: 64-bit-offset MFMA

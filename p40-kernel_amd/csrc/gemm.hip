@@ -1329,6 +1329,11 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
         const int rc = pq2::gemv_small_batch(W, Xq, Y, n_out, n_in, n_tok, stream);
         if (rc >= 0) return rc;
     }
+    // tall matrices at 9 to 16 tokens (its own rule; the small kernels' knobs keep theirs)
+    if (n_tok >= 9 && n_tok <= 16 && knob(pq2host::K_GEMM_SMALL, 0) == 0 && knob(pq2host::K_GEMM_SMALL_CFG, 0) == 0) {
+        const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, gemm_cu_count(), st);
+        if (rc >= 0) return rc;
+    }
     const size_t skinny_lds = (size_t)4 * 16 * PQ2_BYTES * (nb / 4) + 4096;
     const int small_sel = knob(pq2host::K_GEMM_SMALL, 0);   // 0 streamed, 1 previous kernel
     if (off32 && n_tok <= 16 && small_sel == 0 && nb % 2 == 0 && nb >= 8 && ((uintptr_t)W & 3u) == 0 &&

@@ -25,7 +25,9 @@
 // mask, and what that adds to the dot, (1024 + 1) q per code too much, is
 // taken off by the accumulator's start: one MFMA per 16 tokens and chunk with
 // a constant A (-1025, -1028) gives it for every row tile.  All of these are
-// integers below 2^24, so S is exact.
+// integers below 2^24, so S is exact.  80 x 16 tiles, which run batches of up to
+// 16 tokens, start from -1024 and the block's stored sum s instead, as every
+// kernel of those batches does.
 #include <hip/hip_runtime.h>
 
 #include "pq2_device.h"
@@ -83,6 +85,7 @@ __global__ void __launch_bounds__(512)
 gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, float * __restrict__ Y, int n_out,
                 int n_tok, int nb, int tok_tiles) {
     constexpr int BM = 16 * MI, BN = 16 * NI;
+    constexpr bool SUM = NI == 1;                                // batches of up to 16 tokens
     constexpr int WP = BM * 17, WL = (WP + 511) / 512;           // 16-byte pieces of a W step; DMAs per wave
     constexpr int SW = (WP + 63) / 64 * 1024;
     constexpr int RUN = BN * Q81_BYTES / 16;                     // pieces of a run
@@ -164,7 +167,9 @@ gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, 
         uint32_t ex = 0x64006400u, m0 = 0x00030003u, m1 = 0x000C000Cu;
         asm("" : "+v"(ex));
         asm("" : "+s"(m0), "+s"(m1));
-        const v8h fix = as_v8h(0xE401E401u, 0xE401E401u, 0xE404E404u, 0xE404E404u);   // f16 -1025, -1028
+        // f16 -1025 and -1028; with the stored sum taken off instead, -1024 for both
+        const v8h fix = SUM ? as_v8h(0xE400E400u, 0xE400E400u, 0xE400E400u, 0xE400E400u)
+                            : as_v8h(0xE401E401u, 0xE401E401u, 0xE404E404u, 0xE404E404u);
         v4f U[MI][NI];
         // software pipeline over i = (chunk, row tile): while tile i's MFMAs are
         // issued, products LAG MFMAs old are folded and tile i + 1's words read
@@ -213,7 +218,8 @@ gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, 
                     Bf[ni] = q_f16(xw[ni][1], xw[ni][2]);
                     da[c & 1][ni] = f16_bits_to_f32(xw[ni][0] & 0xffffu);
                     asm("" : "+v"(da[c & 1][ni]));              // fp32 from here on, not an f16 source of each FMA
-                    E[ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fix, Bf[ni], (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                    const float ns = SUM ? (float)-((int)xw[ni][0] >> 16) : 0.0f;
+                    E[ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fix, Bf[ni], (v4f){ns, ns, ns, ns}, 0, 0, 0);
                 }
             }
             if (i == MI) {
@@ -299,7 +305,7 @@ int launch_mid(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_out, i
 namespace pq2 {
 
 // Y = W . X where the kernel's requirements hold and it is the faster one; -1:
-// nothing launched.  BONSAI_GEMM_MID: 0 never, 1..6 that tile shape (tests).
+// nothing launched.  BONSAI_GEMM_MID: 0 never, 1..7 that tile shape (tests).
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st) {
     // whole steps of 8 blocks, 16-byte DMA of W's rows, 32-bit offsets (80 rows
     // of W, a block's 4 chunks of X)
@@ -322,7 +328,18 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
     const int forced = pq2host::knob(pq2host::K_GEMM_MID, -1);
     if (forced == 0) return -1;
     if (forced > 0) {
-        pick = (forced < 6 ? forced : 6) - 1;
+        pick = (forced < 7 ? forced : 7) - 1;
+    } else if (n_tok <= 16) {
+        // 9 to 16 tokens: the streamed kernel (gemm_small_kernel) takes 64 rows a CU
+        // and round, 80 x 16 tiles here 80 in the same time, so they are the faster
+        // where their rounds, rounded up, are no more than that one's as a fraction.
+        // Measured (us, streamed -> here, 12 tokens, n_in 5120): 17408 rows 15.5 ->
+        // 13.4, 49152 29.4 -> 28.1, 248320 144 -> 118, 16385x17408 38.1 -> 35.4; on the
+        // other side 10240 rows 9.6 against 10.2, 24576 16.1 against 17.9.  Below 40
+        // blocks this kernel's fp32 sums are no closer to 64 bits than that one's
+        // (17408x3072 6.6e-8 against 6.3e-8; at 5120 7.11e-8 against 7.20e-8).
+        if (nb < 40 || cdiv(n_out, 80 * (int64_t)cus) * 64 * cus > n_out) return -1;
+        pick = 6;
     } else {
         // the 128-row kernel: about 1.0 us a block and round on 64-token tiles,
         // 1.4 us on 128-token ones (gemm_prefill_f16 picks).  Measured (us, that
@@ -342,6 +359,7 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
         case 2: return launch_mid<5, 2>(w, x, Y, n_out, n_tok, nb, st);
         case 3: return launch_mid<4, 2>(w, x, Y, n_out, n_tok, nb, st);
         case 4: return launch_mid<4, 3>(w, x, Y, n_out, n_tok, nb, st);
+        case 6: return launch_mid<5, 1>(w, x, Y, n_out, n_tok, nb, st);
         default: return launch_mid<2, 2>(w, x, Y, n_out, n_tok, nb, st);
     }
 }

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # fp32 sums of nb block terms, each a sum of 4 chunk terms: (nb + 4) roundings of
 # 2^-24 at most, against the largest output; 1e-5 is the bar of every GEMM here
 TOL = 1e-5
-SHAPES = {1: (80, 48), 2: (48, 32), 3: (80, 32), 4: (64, 32), 5: (64, 48), 6: (32, 32)}
+SHAPES = {1: (80, 48), 2: (48, 32), 3: (80, 32), 4: (64, 32), 5: (64, 48), 6: (32, 32), 7: (80, 16)}
 
 
 def normwise(a, ref):
@@ -99,7 +99,7 @@ def test_mid_scales_at_the_ends(knobs):
     assert np.max(np.abs(got[fine] - ref[fine])) <= TOL * np.max(np.abs(ref[fine]))
 
 
-@pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33)])
+@pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33), (17408, 5120, 12)])
 def test_mid_default_dispatch(n_out, n_in, n_tok):
     """Shapes the default rule gives to this kernel, with and without a
     workspace (the same bytes), on a row sample."""
@@ -118,3 +118,20 @@ def test_mid_default_dispatch(n_out, n_in, n_tok):
     Ws = np.concatenate([W[r * rb:(r + 1) * rb] for r in rows])
     assert np.all(np.isfinite(got))
     assert normwise(got[rows], O.gemm(Ws, Xq, rows.size, n_in, n_tok, nthreads=16)) <= TOL
+
+
+def test_mid_stored_sum_up_to_16_tokens(knobs):
+    """Batches of up to 16 tokens subtract each activation block's stored s,
+    whatever it is: the 80 x 16 tiles as the streamed kernel of those sizes, and
+    as the reference."""
+    n_out, n_in, n_tok = 83, 5120, 13
+    case(f"mid GEMM {n_out}x{n_in}x{n_tok}, stored sums that are not the sums")
+    W = O.gen_weights(6500, n_out, n_in)
+    Xq = O.quantize_chunk_major(O.gen_normal(6501, n_tok * n_in).reshape(n_tok, n_in)).copy()
+    s = np.random.default_rng(65).integers(-32768, 32768, Xq.size // 36, dtype=np.int16)
+    Xq.reshape(-1, 36)[:, 2:4] = s.view(np.uint8).reshape(-1, 2)
+    Wd, Xd = dev(W), dev(Xq)
+    ref = O.gemm(W, Xq, n_out, n_in, n_tok, nthreads=16)
+    for knob in (7, 0):
+        knobs.set("BONSAI_GEMM_MID", knob)
+        assert normwise(gemm(Wd, Xd, n_out, n_in, n_tok), ref) <= TOL
