@@ -1242,3 +1242,31 @@ def test_rms_prepass_tokens_equal_single_rows(n, n_tok):
         B.rmsnorm_fwht_quant(x[t * n:(t + 1) * n], w, signs, row, n, 1, 1e-6)
         rows.append(host(row).reshape(-1, 36))
     np.testing.assert_array_equal(host(got).reshape(n // 32, n_tok, 36), np.stack(rows, axis=1))
+
+
+@pytest.mark.parametrize("n_out,n_in,n_tok", [(19, 17408, 9), (1024, 5120, 12), (4096, 5120, 13), (4097, 6144, 16),
+                                              (8191, 5120, 12), (8193, 5120, 10), (5120, 4992, 12)])
+def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok):
+    """9..16 tokens on the streamed kernel at the edges of its workgroup shapes
+    (16 rows with K split 8 ways, 32 rows past one round of those, 16 rows with
+    K split 4 ways past one round of these and on short rows) and of its rings
+    (12 and 16 tokens): against the oracle on the first, middle and last rows,
+    and against one GEMV per token."""
+    case(f"gemm streamed {n_out}x{n_in}x{n_tok}")
+    W = O.gen_weights(1800 + n_out + n_tok, n_out, n_in)
+    Xq = O.quantize_chunk_major(O.gen_normal(1801 + n_in, n_tok * n_in).reshape(n_tok, n_in))
+    Wd = dev(W)
+    Y = torch.full((n_out, n_tok), float("nan"), dtype=torch.float32, device="cuda")
+    B.gemm(Wd, dev(Xq), Y, n_out, n_in, n_tok)
+    got = host(Y)
+    assert np.all(np.isfinite(got))
+    rows = sorted(set(range(min(n_out, 40))) | set(range(n_out // 2, min(n_out, n_out // 2 + 16))) |
+                  set(range(max(0, n_out - 40), n_out)))
+    rb = n_in // 128 * 34
+    Ws = np.concatenate([W[r * rb:(r + 1) * rb] for r in rows])
+    assert normwise(got[rows], O.gemm(Ws, Xq, len(rows), n_in, n_tok, nthreads=16)) <= TOL
+    for t in range(n_tok):
+        xt = np.ascontiguousarray(Xq.reshape(n_in // 32, n_tok, 36)[:, t]).reshape(-1)
+        y = torch.full((n_out,), float("nan"), dtype=torch.float32, device="cuda")
+        B.gemv(Wd, dev(xt), y, n_out, n_in)
+        assert normwise(got[:, t], host(y)) <= 2 * TOL
