@@ -317,10 +317,11 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
         int mi, ni;
         float us;
     };
-    static constexpr Shape shapes[6] = {{5, 3, 3.6f}, {3, 2, 1.8f}, {5, 2, 2.5f}, {4, 2, 2.05f}, {4, 3, 2.8f}, {2, 2, 1.45f}};
+    static constexpr Shape shapes[7] = {{5, 3, 3.6f}, {3, 2, 1.8f}, {5, 2, 2.5f}, {4, 2, 2.05f},
+                                        {4, 3, 2.8f}, {2, 2, 1.45f}, {5, 1, 1.9f}};
     int pick = 0;
     float best = 0.0f;
-    for (int k = 0; k < 6; ++k) {
+    for (int k = 0; k < 6; ++k) {                              // the last: up to 16 tokens, below
         const int64_t wgs = cdiv(n_out, 16 * shapes[k].mi) * cdiv(n_tok, 16 * shapes[k].ni);
         const float t = 4.0f + (float)cdiv(wgs, cus) * (float)(nb / 8) * shapes[k].us;
         if (k == 0 || t < best) best = t, pick = k;
