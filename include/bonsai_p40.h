@@ -67,9 +67,9 @@ int bonsai_p40_quant_activations(const float * x, void * out, int64_t n, bonsai_
 // kernel; 9..16 the streamed 16x16x32 int8 MFMA kernel, or on tall matrices
 // (17408 rows) f16-MFMA 80x16 tiles that read s as it does; larger n_tok the
 // f16-MFMA tile GEMMs: small tiles with K split over a workgroup's waves
-// where larger ones would leave CUs idle (n_in % 1024 == 0, 16-byte aligned
-// W), else 128- to 256-row tiles (other alignments: 64-bit-offset MFMA
-// kernels).  The GEMV and the streamed small-batch kernels subtract each Q8_1
+// where larger ones would leave CUs idle, for all tokens or those past the
+// whole larger tiles (n_in % 1024 == 0, 16-byte aligned W), else 128- to
+// 256-row tiles (other alignments: 64-bit-offset MFMA kernels).  The GEMV and the streamed small-batch kernels subtract each Q8_1
 // block's stored sum s as the reference does (src/pq2_0.h:169); the tile GEMMs
 // and the kernels for other alignments multiply (code - 1) by q directly and
 // do not read s.  The two agree for blocks whose s is the sum of their q, which

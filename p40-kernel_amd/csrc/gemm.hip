@@ -1233,9 +1233,10 @@ gemm_f16_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X,
         }
 }
 
-// The 128-row f16 prefill kernel (gemm_f16_kernel) over rows [0, n_out) of w / Y.
+// The 128-row f16 prefill kernel (gemm_f16_kernel) over rows [0, n_out) of w / Y
+// and tokens [0, cols), cols a multiple of 128 or n_tok.
 int gemm_prefill_f16(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_out, int64_t n_tok, int nb,
-                     hipStream_t st) {
+                     int64_t cols, hipStream_t st) {
     // 16 waves (4 per SIMD, 32 x 32 wave tiles) measured 12-22 % faster than
     // 8 waves (2 per SIMD, 64 x 32) on every prefill shape: the latency of
     // the chunk pipeline and the per-block barrier is hidden by more waves.
@@ -1243,7 +1244,7 @@ int gemm_prefill_f16(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_
     // one round, 64-token tiles put twice the CUs to work (6144x5120 at
     // M = 256: 61 -> 42 us); past that the extra round costs more than the
     // idle CUs (5120x17408 at M = 512: 200 -> 256 us), so 128.
-    const int64_t tiles128 = cdiv(n_out, GF_BM) * cdiv(n_tok, 128);
+    const int64_t tiles128 = cdiv(n_out, GF_BM) * cdiv(cols, 128);
     int bn = knob(pq2host::K_GEMM_F16_BN, 0);
     if (bn != 64 && bn != 128) bn = 2 * tiles128 <= gemm_cu_count() ? 64 : 128;
     // A last round that only part-fills the CUs (17408 rows at M = 512:
@@ -1252,24 +1253,24 @@ int gemm_prefill_f16(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_
     // remaining rows as a second launch of 64-token tiles, which spreads
     // them over more CUs (twice the tiles, each about half the work).
     const int cus = gemm_cu_count();
-    const int64_t ttok = cdiv(n_tok, 128), rounds = tiles128 / cus, rest = tiles128 - rounds * cus;
+    const int64_t ttok = cdiv(cols, 128), rounds = tiles128 / cus, rest = tiles128 - rounds * cus;
     if (bn == 128 && rounds >= 1 && rest > 0 && 2 * rest <= cus && (rounds * cus) % ttok == 0 &&
         knob(pq2host::K_GEMM_F16_SPLIT, 1) > 0 && knob(pq2host::K_GEMM_F16_WAVES, 16) != 8) {
         const int64_t rows_main = rounds * cus / ttok * GF_BM;
         const int64_t rows_tail = n_out - rows_main;
-        if (rows_tail > 0 && cdiv(rows_tail, GF_BM) * cdiv(n_tok, 64) <= cus) {
+        if (rows_tail > 0 && cdiv(rows_tail, GF_BM) * cdiv(cols, 64) <= cus) {
             hipLaunchKernelGGL((gemm_f16_kernel<4, 4, 2, 2>), dim3((unsigned)(rows_main / GF_BM), (unsigned)ttok),
                                dim3(1024), 0, st, w, x, Y, (int)rows_main, (int)n_tok, nb);
             hipLaunchKernelGGL((gemm_f16_kernel<4, 4, 2, 1, 64>),
-                               dim3((unsigned)cdiv(rows_tail, GF_BM), (unsigned)cdiv(n_tok, 64)), dim3(1024), 0,
+                               dim3((unsigned)cdiv(rows_tail, GF_BM), (unsigned)cdiv(cols, 64)), dim3(1024), 0,
                                st, w + (size_t)rows_main * PQ2_BYTES * nb, x, Y + (size_t)rows_main * n_tok,
                                (int)rows_tail, (int)n_tok, nb);
             return (int)hipGetLastError();
         }
     }
-    const dim3 grid((unsigned)cdiv(n_out, GF_BM), (unsigned)cdiv(n_tok, bn));
+    const dim3 grid((unsigned)cdiv(n_out, GF_BM), (unsigned)cdiv(cols, bn));
     if (knob(pq2host::K_GEMM_F16_WAVES, 16) == 8)
-        hipLaunchKernelGGL((gemm_f16_kernel<2, 4, 4, 2>), dim3(grid.x, (unsigned)cdiv(n_tok, 128)), dim3(512),
+        hipLaunchKernelGGL((gemm_f16_kernel<2, 4, 4, 2>), dim3(grid.x, (unsigned)cdiv(cols, 128)), dim3(512),
                            0, st, w, x, Y, (int)n_out, (int)n_tok, nb);
     else if (bn == 64)
         hipLaunchKernelGGL((gemm_f16_kernel<4, 4, 2, 1, 64>), grid, dim3(1024), 0, st, w, x, Y, (int)n_out,
@@ -1288,16 +1289,68 @@ int gemv_small_batch(const void * W, const void * Xq, float * Y, int64_t n_out, 
 // gemm_wide.hip: rows [0, rows) that the wide kernel takes (0: none) and its launch
 int64_t gemm_wide_rows(const void * W, const void * Xq, int64_t n_out, int64_t n_tok, int nb, int cus, bool force,
                        int * mi);
-int gemm_wide_launch(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
-                     hipStream_t st);
 int64_t gemm_wide_x16_bytes(int64_t n_tok, int nb);
+int gemm_wide_launch(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int64_t cols,
+                     int mi, hipStream_t st);
+int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int64_t cols,
+                        int mi, void * ws, hipStream_t st);
 // gemm_mid.hip: small tiles with K split over a workgroup's waves; -1 if not applicable
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st);
-int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
-                        void * ws, hipStream_t st);
+float gemm_mid_us(const void * W, int64_t n_out, int64_t first, int64_t n_tok, int nb, int cus);
+int gemm_mid_tail(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb,
+                  int cus, hipStream_t st);
 }
 
 namespace {
+
+// Time (us) of tokens [0, cols) on the large tiles, rows as gemm_wide_rows
+// gives them: rounds of workgroups times what a round takes a block of K
+// (MI355X: 4.5 us on 256-row tiles, 3.45 on 160-row ones, 1.42 on 128 x 128,
+// 1.05 on 128 x 64)
+float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows, int mi) {
+    float us = 0.0f;
+    if (rows > 0) us = (mi == 8 ? 4.5f : 3.45f) * (float)cdiv(cdiv(rows, 32 * mi) * cdiv(cols, 256), cus);
+    if (rows < n_out) {
+        // gemm_prefill_f16's choice
+        const int64_t R = cdiv(n_out - rows, GF_BM), T = cdiv(cols, 128), full = R * T / cus, rest = R * T - full * cus;
+        if (2 * R * T <= cus) us += 1.05f;
+        else if (full >= 1 && rest > 0 && 2 * rest <= cus && full * cus % T == 0 && (R - full * cus / T) * cdiv(cols, 64) <= cus)
+            us += 1.42f * (float)full + 1.05f;
+        else us += 1.42f * (float)cdiv(R * T, cus);
+    }
+    return us * (float)nb;
+}
+
+// The tiles of a prefill: tokens [0, cols) on the large ones, the first rows of
+// them on the wide kernel (tile height mi), tokens [cols, n_tok) on the small
+// ones (gemm_mid.hip; cols = 0: all of them).  rows and mi come as
+// gemm_wide_rows gives them for every token; another plan has to be 5 % faster
+// by its estimate.  Small tiles take over the whole product where large ones
+// would leave most CUs idle, or the tokens past the whole large tiles where
+// these would start another round, and rows whose wide tiles are short of a round
+// take 128-row tiles where those have fewer empty tokens.  Measured (us, large
+// tiles as gemm_wide_rows has them -> this plan): 17408x5120 with 20 tokens 57
+// -> 17, 33 54 -> 22, 140 101 -> 63, 400 159 -> 126; 5120x17408 with 100 132 ->
+// 45, 800 361 -> 213; 10240x5120 with 386 102 -> 69, 777 139 -> 132 (768 + 9
+// tokens), 1166 229 -> 180; unchanged 17408x5120 with 1500, 10240x5120 with 1900.
+void prefill_plan(const void * W, const void * Xq, int64_t n_out, int64_t n_tok, int nb, int cus, int64_t * cols,
+                  int64_t * rows, int * mi) {
+    float best = 0.95f * large_us(n_out, n_tok, nb, cus, *rows, *mi);
+    const float small = pq2::gemm_mid_us(W, n_out, 0, n_tok, nb, cus);
+    if (small > 0.0f && small < best) best = small, *cols = 0, *rows = 0;
+    // gemm_wide_rows looks at the tokens that it is given only
+    if ((uint64_t)n_tok * Q81_BYTES * 4ull * (uint64_t)nb >= (1ull << 31)) return;
+    for (int64_t c : {n_tok, n_tok / 128 * 128, n_tok / 256 * 256}) {
+        float us = 0.0f;
+        if (c < n_tok) us = pq2::gemm_mid_us(W, n_out, c, n_tok, nb, cus);
+        if (c == 0 || (c < n_tok && us == 0.0f)) continue;
+        int m = 8;
+        const int64_t r = pq2::gemm_wide_rows(W, Xq, n_out, c, nb, cus, false, &m);
+        const float wide = us + large_us(n_out, c, nb, cus, r, m), plain = us + large_us(n_out, c, nb, cus, 0, 8);
+        if (r > 0 && (c == n_tok || c % 256 == 0) && wide < best) best = wide, *cols = c, *rows = r, *mi = m;
+        if (plain < best) best = plain, *cols = c, *rows = 0;
+    }
+}
 
 // bonsai_p40_gemm's dispatch; ws (non-NULL: large enough and aligned, checked
 // by the caller) lets the long-prompt kernel take the activation by DMA
@@ -1376,32 +1429,35 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
     if (knob(pq2host::K_GEMM_KERNEL, 0) == 0) {
         // long prompts: the 256-row wide kernel (gemm_wide.hip) over the rows
         // whose tiles fill whole rounds of CUs, the 128-row kernel for the rest
-        const int wide = knob(pq2host::K_GEMM_WIDE, 1);
-        if (wide != 0 && n_tok > 16) {
-            int mi = 8;
-            const int64_t rows = pq2::gemm_wide_rows(W, Xq, n_out, n_tok, nb, gemm_cu_count(), wide == 2, &mi);
-            if (rows > 0) {
-                // with a workspace: the activation converted once (an extra
-                // pass of 100 B per Q8_1 block), then the tiles DMA it -- worth
-                // it where that pass is spread over enough rows (measured on
-                // MI355X, M = 2048: 17408x5120 425 -> 414 us, 5120x17408 450 ->
-                // 459 us, so 8192 rows and more)
-                const bool via_ws = ws != nullptr && n_out >= 8192;
-                const int rc = via_ws ? pq2::gemm_wide_launch_ws(W, Xq, Y, rows, n_tok, nb, mi, ws, st)
-                                      : pq2::gemm_wide_launch(W, Xq, Y, rows, n_tok, nb, mi, st);
-                if (rc != 0 || rows == n_out) return rc;
-                return gemm_prefill_f16(w + (size_t)rows * PQ2_BYTES * nb, x, Y + (size_t)rows * n_tok,
-                                        n_out - rows, n_tok, nb, st);
-            }
-        }
-        // what the wide kernel leaves: small tiles where 128-row tiles would
-        // leave most CUs idle (BONSAI_GEMM_WIDE other than 1 compares the tile
-        // kernels, which add in one order)
-        if (wide == 1 || knob(pq2host::K_GEMM_MID, -1) > 0) {
-            const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, gemm_cu_count(), st);
+        const int wide = n_tok > 16 ? knob(pq2host::K_GEMM_WIDE, 1) : 0;
+        const int cus = gemm_cu_count();
+        int mi = 8;
+        int64_t cols = n_tok;                                   // tokens of the large tiles; the rest on small ones
+        int64_t rows = wide != 0 ? pq2::gemm_wide_rows(W, Xq, n_out, n_tok, nb, cus, wide == 2, &mi) : 0;
+        // (BONSAI_GEMM_WIDE other than 1 compares the large tiles, which add in one
+        // order; BONSAI_GEMM_MID forces a small one)
+        if (knob(pq2host::K_GEMM_MID, -1) > 0) {
+            const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, cus, st);
             if (rc >= 0) return rc;
+        } else if (wide == 1) {
+            prefill_plan(W, Xq, n_out, n_tok, nb, cus, &cols, &rows, &mi);
         }
-        return gemm_prefill_f16(w, x, Y, n_out, n_tok, nb, st);
+        int rc = 0;
+        if (rows > 0) {
+            // with a workspace: the activation converted once (an extra
+            // pass of 100 B per Q8_1 block), then the tiles DMA it -- worth
+            // it where that pass is spread over enough rows (measured on
+            // MI355X, M = 2048: 17408x5120 425 -> 414 us, 5120x17408 450 ->
+            // 459 us, so 8192 rows and more)
+            const bool via_ws = ws != nullptr && n_out >= 8192;
+            rc = via_ws ? pq2::gemm_wide_launch_ws(W, Xq, Y, rows, n_tok, nb, cols, mi, ws, st)
+                        : pq2::gemm_wide_launch(W, Xq, Y, rows, n_tok, nb, cols, mi, st);
+        }
+        if (rc == 0 && cols > 0 && rows < n_out)
+            rc = gemm_prefill_f16(w + (size_t)rows * PQ2_BYTES * nb, x, Y + (size_t)rows * n_tok, n_out - rows, n_tok,
+                                  nb, cols, st);
+        if (rc == 0 && cols < n_tok) rc = pq2::gemm_mid_tail(W, Xq, Y, n_out, cols, n_tok, nb, cus, st);
+        return rc;
     } else if ((nb & 1) || ((uintptr_t)W & 3u) != 0) {
         dim3 grid((unsigned)cdiv(n_out, 64), (unsigned)cdiv(n_tok, 64));
         hipLaunchKernelGGL(gemm_mfma_kernel_u16, grid, dim3(256), 0, st, w, x, Y, (int)n_out, (int)n_tok, nb);

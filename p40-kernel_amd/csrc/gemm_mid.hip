@@ -35,6 +35,7 @@
 #include "../../include/bonsai_p40.h"
 
 #include <stdint.h>
+#include <algorithm>
 
 using namespace pq2;
 
@@ -80,12 +81,11 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint8_t * to, ui
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)to, 16, off, soff, 0, 0);
 }
 
-template <int MI, int NI>
+template <int MI, int NI, bool SUM>
 __global__ void __launch_bounds__(512)
 gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, float * __restrict__ Y, int n_out,
-                int n_tok, int nb, int tok_tiles) {
+                int n_tok, int nb, int tok_first, int tok_tiles) {
     constexpr int BM = 16 * MI, BN = 16 * NI;
-    constexpr bool SUM = NI == 1;                                // batches of up to 16 tokens
     constexpr int WP = BM * 17, WL = (WP + 511) / 512;           // 16-byte pieces of a W step; DMAs per wave
     constexpr int SW = (WP + 63) / 64 * 1024;
     constexpr int RUN = BN * Q81_BYTES / 16;                     // pieces of a run
@@ -104,7 +104,7 @@ gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, 
     // token tiles of one row tile next to each other: they share W in its L2
     const int total = gridDim.x, xcd = blockIdx.x & 7;
     const int tile = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
-    const int row0 = tile / tok_tiles * BM, tok0 = tile % tok_tiles * BN;
+    const int row0 = tile / tok_tiles * BM, tok0 = tok_first + tile % tok_tiles * BN;
 
     const uint32_t rs = (uint32_t)PQ2_BYTES * nb;
     uint32_t w_off[WL];
@@ -292,44 +292,79 @@ gemm_mid_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X, 
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-template <int MI, int NI>
-int launch_mid(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_out, int64_t n_tok, int nb, hipStream_t st) {
-    const int64_t R = cdiv(n_out, 16 * MI), T = cdiv(n_tok, 16 * NI);
-    hipLaunchKernelGGL((gemm_mid_kernel<MI, NI>), dim3((unsigned)(R * T)), dim3(512), 0, st, w, x, Y, (int)n_out,
-                       (int)n_tok, nb, (int)T);
+template <int MI, int NI, bool SUM = false>
+int launch_mid(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb,
+               hipStream_t st) {
+    const int64_t R = cdiv(n_out, 16 * MI), T = cdiv(n_tok - first, 16 * NI);
+    hipLaunchKernelGGL((gemm_mid_kernel<MI, NI, SUM>), dim3((unsigned)(R * T)), dim3(512), 0, st, w, x, Y, (int)n_out,
+                       (int)n_tok, nb, (int)first, (int)T);
     return (int)hipGetLastError();
+}
+
+// Tile shapes, and per shape the time of one step on one CU (MI355X, us, the
+// slope over K of one round of workgroups); a CU holds one workgroup, a launch
+// starts and reduces in about 4 us, and many full rounds lower the clock
+// (17408x5120 with 400 tokens: 8 rounds of 80 x 48 in 171 us, 33 tokens: one in 22).  80 x 16 tiles that read the stored
+// sums run batches of up to 16 tokens only.
+struct Shape {
+    int mi, ni;
+    float us;
+    bool sum;
+};
+constexpr int SHAPES = 9, SHAPE_SUM = 6;
+constexpr Shape shapes[SHAPES] = {{5, 3, 3.6f, false},  {3, 2, 1.8f, false}, {5, 2, 2.5f, false},
+                                  {4, 2, 2.05f, false}, {4, 3, 2.8f, false}, {2, 2, 1.45f, false},
+                                  {5, 1, 1.9f, true},   {5, 1, 1.8f, false}, {3, 1, 1.2f, false}};
+
+// The fastest shape for n_tok tokens, and its time
+int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus, float * us) {
+    int pick = -1;
+    for (int k = 0; k < SHAPES; ++k) {
+        if (shapes[k].sum) continue;
+        const int64_t wgs = cdiv(n_out, 16 * shapes[k].mi) * cdiv(n_tok, 16 * shapes[k].ni);
+        const float r = (float)cdiv(wgs, cus), t = 4.0f + r * (1.0f + 0.02f * std::min(r, 8.0f)) * (float)(nb / 8) * shapes[k].us;
+        if (pick < 0 || t < *us) *us = t, pick = k;
+    }
+    return pick;
+}
+
+// Whole steps of 8 blocks, 16-byte DMA of W's rows, 32-bit offsets (80 rows of
+// W, a block's 4 chunks of X), a grid of under 2^32 threads
+bool mid_takes(const void * W, int64_t n_out, int64_t n_tok, int nb) {
+    return nb % 8 == 0 && ((uintptr_t)W & 15u) == 0 && nb <= (1 << 20) && n_tok <= (1 << 24) &&
+           cdiv(n_out, 32) * cdiv(n_tok, 16) <= (1 << 22);
+}
+
+int run_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb, int pick,
+            hipStream_t st) {
+    const uint8_t * w = (const uint8_t *)W, * x = (const uint8_t *)Xq;
+    switch (pick) {
+        case 0: return launch_mid<5, 3>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 1: return launch_mid<3, 2>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 2: return launch_mid<5, 2>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 3: return launch_mid<4, 2>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 4: return launch_mid<4, 3>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 5: return launch_mid<2, 2>(w, x, Y, n_out, first, n_tok, nb, st);
+        case SHAPE_SUM: return launch_mid<5, 1, true>(w, x, Y, n_out, first, n_tok, nb, st);
+        case 7: return launch_mid<5, 1>(w, x, Y, n_out, first, n_tok, nb, st);
+        default: return launch_mid<3, 1>(w, x, Y, n_out, first, n_tok, nb, st);
+    }
 }
 
 }  // namespace
 
 namespace pq2 {
 
-// Y = W . X where the kernel's requirements hold and it is the faster one; -1:
-// nothing launched.  BONSAI_GEMM_MID: 0 never, 1..7 that tile shape (tests).
+// Y = W . X of up to 16 tokens where the kernel's requirements hold and it is
+// the faster one; -1: nothing launched.  BONSAI_GEMM_MID: 0 never, 1..9 that tile
+// shape, whatever the tokens (tests).
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st) {
-    // whole steps of 8 blocks, 16-byte DMA of W's rows, 32-bit offsets (80 rows
-    // of W, a block's 4 chunks of X)
-    if (nb % 8 != 0 || nb > (1 << 20) || n_tok > (1 << 24) || ((uintptr_t)W & 15u) != 0) return -1;
-    // Per tile shape the time of one step on one CU (MI355X, us, the slope
-    // over K of one round of workgroups); a CU holds one workgroup, and a
-    // launch starts and reduces in about 4 us.
-    struct Shape {
-        int mi, ni;
-        float us;
-    };
-    static constexpr Shape shapes[7] = {{5, 3, 3.6f}, {3, 2, 1.8f}, {5, 2, 2.5f}, {4, 2, 2.05f},
-                                        {4, 3, 2.8f}, {2, 2, 1.45f}, {5, 1, 1.9f}};
-    int pick = 0;
-    float best = 0.0f;
-    for (int k = 0; k < 6; ++k) {                              // the last: up to 16 tokens, below
-        const int64_t wgs = cdiv(n_out, 16 * shapes[k].mi) * cdiv(n_tok, 16 * shapes[k].ni);
-        const float t = 4.0f + (float)cdiv(wgs, cus) * (float)(nb / 8) * shapes[k].us;
-        if (k == 0 || t < best) best = t, pick = k;
-    }
     const int forced = pq2host::knob(pq2host::K_GEMM_MID, -1);
-    if (forced == 0) return -1;
+    if (forced == 0 || !mid_takes(W, n_out, n_tok, nb)) return -1;
+    float us = 0.0f;
+    int pick = mid_pick(n_out, n_tok, nb, cus, &us);
     if (forced > 0) {
-        pick = (forced < 7 ? forced : 7) - 1;
+        pick = (forced < SHAPES ? forced : SHAPES) - 1;
     } else if (n_tok <= 16) {
         // 9 to 16 tokens: the streamed kernel (gemm_small_kernel) takes 64 rows a CU
         // and round, 80 x 16 tiles here 80 in the same time, so they are the faster
@@ -340,29 +375,27 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
         // blocks this kernel's fp32 sums are no closer to 64 bits than that one's
         // (17408x3072 6.6e-8 against 6.3e-8; at 5120 7.11e-8 against 7.20e-8).
         if (nb < 40 || cdiv(n_out, 80 * (int64_t)cus) * 64 * cus > n_out) return -1;
-        pick = 6;
+        pick = SHAPE_SUM;
     } else {
-        // the 128-row kernel: about 1.0 us a block and round on 64-token tiles,
-        // 1.4 us on 128-token ones (gemm_prefill_f16 picks).  Measured (us, that
-        // kernel -> this one): 17408x5120 with 20 tokens 57 -> 17, 33 56 -> 22, 96
-        // 56 -> 41, but 128 57 -> 60; 5120x17408 with 32 tokens 129 -> 28, 100
-        // 132 -> 47, 256 134 -> 90; 1024x5120 with 512 tokens 42 -> 14.
-        const int64_t t128 = cdiv(n_out, 128) * cdiv(n_tok, 128);
-        const bool b64 = 2 * t128 <= cus;
-        const float other = (float)nb * (b64 ? 1.0f : 1.4f * (float)cdiv(t128, cus));
-        if (best > 0.9f * other) return -1;
+        return -1;                                             // gemm_dispatch's plan
     }
-    if (cdiv(n_out, 16 * shapes[pick].mi) * cdiv(n_tok, 16 * shapes[pick].ni) > (1 << 22)) return -1;   // 512 threads each
-    const uint8_t * w = (const uint8_t *)W, * x = (const uint8_t *)Xq;
-    switch (pick) {
-        case 0: return launch_mid<5, 3>(w, x, Y, n_out, n_tok, nb, st);
-        case 1: return launch_mid<3, 2>(w, x, Y, n_out, n_tok, nb, st);
-        case 2: return launch_mid<5, 2>(w, x, Y, n_out, n_tok, nb, st);
-        case 3: return launch_mid<4, 2>(w, x, Y, n_out, n_tok, nb, st);
-        case 4: return launch_mid<4, 3>(w, x, Y, n_out, n_tok, nb, st);
-        case 6: return launch_mid<5, 1>(w, x, Y, n_out, n_tok, nb, st);
-        default: return launch_mid<2, 2>(w, x, Y, n_out, n_tok, nb, st);
-    }
+    return run_mid(W, Xq, Y, n_out, 0, n_tok, nb, pick, st);
+}
+
+// Estimated time (us) of tokens [first, n_tok) here; 0 where the kernel does
+// not take them
+float gemm_mid_us(const void * W, int64_t n_out, int64_t first, int64_t n_tok, int nb, int cus) {
+    float us = 0.0f;
+    if (pq2host::knob(pq2host::K_GEMM_MID, -1) < 0 && mid_takes(W, n_out, n_tok, nb))
+        mid_pick(n_out, n_tok - first, nb, cus, &us);
+    return us;
+}
+
+// Tokens [first, n_tok) of the product (gemm_mid_us takes them)
+int gemm_mid_tail(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb,
+                  int cus, hipStream_t st) {
+    float us = 0.0f;
+    return run_mid(W, Xq, Y, n_out, first, n_tok, nb, mid_pick(n_out, n_tok - first, nb, cus, &us), st);
 }
 
 }  // namespace pq2

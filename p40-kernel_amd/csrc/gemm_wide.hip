@@ -569,10 +569,11 @@ int64_t gemm_wide_rows(const void * W, const void * Xq, int64_t n_out, int64_t n
 }
 
 // The wide kernel (mi = 8 or 5) over rows [0, n_out) of W / Y (the caller
-// offsets both for a row range); requires what gemm_wide_rows checks.
-int gemm_wide_launch(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
-                     hipStream_t st) {
-    const unsigned gy = (unsigned)((n_tok + WB_N - 1) / WB_N);
+// offsets both for a row range) and tokens [0, cols), cols a multiple of 256 or
+// n_tok; requires what gemm_wide_rows checks.
+int gemm_wide_launch(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int64_t cols,
+                     int mi, hipStream_t st) {
+    const unsigned gy = (unsigned)((cols + WB_N - 1) / WB_N);
     const uint8_t * w = (const uint8_t *)W, * x = (const uint8_t *)Xq;
     if (mi == 5)
         hipLaunchKernelGGL((gemm_wide_kernel<5, false>), dim3((unsigned)((n_out + 159) / 160), gy), dim3(512), 0, st,
@@ -595,14 +596,14 @@ int64_t gemm_wide_x16_bytes(int64_t n_tok, int nb) {
 // The same product as gemm_wide_launch, with the activation converted once
 // into ws (gemm_wide_x16_bytes, 16-byte aligned) and the kernel's B side
 // arriving by LDS-DMA from there; bit-identical to gemm_wide_launch.
-int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int mi,
-                        void * ws, hipStream_t st) {
+int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int64_t cols,
+                        int mi, void * ws, hipStream_t st) {
     const int64_t blocks = n_tok * 4 * (int64_t)nb;
     uint8_t * x16 = static_cast<uint8_t *>(ws);
     float * xd = reinterpret_cast<float *>(x16 + blocks * 64);
     hipLaunchKernelGGL(wide_x16_kernel, dim3((unsigned)((2 * blocks + 255) / 256)), dim3(256), 0, st,
                        (const uint8_t *)Xq, x16, xd, blocks);
-    const unsigned gy = (unsigned)((n_tok + WB_N - 1) / WB_N);
+    const unsigned gy = (unsigned)((cols + WB_N - 1) / WB_N);
     const uint8_t * w = (const uint8_t *)W, * x = (const uint8_t *)Xq;
     if (mi == 5)
         hipLaunchKernelGGL((gemm_wide_kernel<5, true>), dim3((unsigned)((n_out + 159) / 160), gy), dim3(512), 0, st,

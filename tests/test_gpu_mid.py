@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # fp32 sums of nb block terms, each a sum of 4 chunk terms: (nb + 4) roundings of
 # 2^-24 at most, against the largest output; 1e-5 is the bar of every GEMM here
 TOL = 1e-5
-SHAPES = {1: (80, 48), 2: (48, 32), 3: (80, 32), 4: (64, 32), 5: (64, 48), 6: (32, 32), 7: (80, 16)}
+SHAPES = {1: (80, 48), 2: (48, 32), 3: (80, 32), 4: (64, 32), 5: (64, 48), 6: (32, 32), 7: (80, 16), 8: (80, 16), 9: (48, 16)}
 
 
 def normwise(a, ref):
@@ -99,10 +99,12 @@ def test_mid_scales_at_the_ends(knobs):
     assert np.max(np.abs(got[fine] - ref[fine])) <= TOL * np.max(np.abs(ref[fine]))
 
 
-@pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33), (17408, 5120, 12)])
+@pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33), (17408, 5120, 12),
+                                              (6144, 5120, 651), (10240, 5120, 777), (17408, 5120, 400)])
 def test_mid_default_dispatch(n_out, n_in, n_tok):
-    """Shapes the default rule gives to this kernel, with and without a
-    workspace (the same bytes), on a row sample."""
+    """Shapes the default rule gives to this kernel, whole or the tokens past the
+    large tiles' whole ones, with and without a workspace (the same bytes), on a
+    row sample."""
     case(f"mid GEMM by default: {n_out}x{n_in}x{n_tok}")
     W = O.gen_weights(6400 + n_out, n_out, n_in)
     X = O.gen_normal(6401 + n_tok, n_tok * n_in).reshape(n_tok, n_in)
