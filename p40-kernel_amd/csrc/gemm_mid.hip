@@ -316,13 +316,15 @@ constexpr Shape shapes[SHAPES] = {{5, 3, 3.6f, false},  {3, 2, 1.8f, false}, {5,
                                   {4, 2, 2.05f, false}, {4, 3, 2.8f, false}, {2, 2, 1.45f, false},
                                   {5, 1, 1.9f, true},   {5, 1, 1.8f, false}, {3, 1, 1.2f, false}};
 
-// The fastest shape for n_tok tokens, and its time
+// The fastest shape for n_tok tokens, and its time (mid_takes first: 32-bit
+// arithmetic, this runs on every call)
 int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus, float * us) {
     int pick = -1;
     for (int k = 0; k < SHAPES; ++k) {
         if (shapes[k].sum) continue;
-        const int64_t wgs = cdiv(n_out, 16 * shapes[k].mi) * cdiv(n_tok, 16 * shapes[k].ni);
-        const float r = (float)cdiv(wgs, cus), t = 4.0f + r * (1.0f + 0.02f * std::min(r, 8.0f)) * (float)(nb / 8) * shapes[k].us;
+        const uint32_t bm = 16 * shapes[k].mi, bn = 16 * shapes[k].ni;
+        const uint32_t wgs = (((uint32_t)n_out + bm - 1) / bm) * (((uint32_t)n_tok + bn - 1) / bn);
+        const float r = (float)((wgs + (uint32_t)cus - 1) / (uint32_t)cus), t = 4.0f + r * (1.0f + 0.02f * std::min(r, 8.0f)) * (float)(nb / 8) * shapes[k].us;
         if (pick < 0 || t < *us) *us = t, pick = k;
     }
     return pick;
@@ -360,12 +362,11 @@ namespace pq2 {
 // shape, whatever the tokens (tests).
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st) {
     const int forced = pq2host::knob(pq2host::K_GEMM_MID, -1);
-    if (forced == 0 || !mid_takes(W, n_out, n_tok, nb)) return -1;
-    float us = 0.0f;
-    int pick = mid_pick(n_out, n_tok, nb, cus, &us);
+    int pick = SHAPE_SUM;
     if (forced > 0) {
         pick = (forced < SHAPES ? forced : SHAPES) - 1;
-    } else if (n_tok <= 16) {
+    } else if (forced == 0 || n_tok > 16 || nb < 40 || n_out <= 64 * (int64_t)cus ||
+               cdiv(n_out, 80 * (int64_t)cus) * 64 * cus > n_out) {
         // 9 to 16 tokens: the streamed kernel (gemm_small_kernel) takes 64 rows a CU
         // and round, 80 x 16 tiles here 80 in the same time, so they are the faster
         // where their rounds, rounded up, are no more than that one's as a fraction.
@@ -373,12 +374,11 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
         // 13.4, 49152 29.4 -> 28.1, 248320 144 -> 118, 16385x17408 38.1 -> 35.4; on the
         // other side 10240 rows 9.6 against 10.2, 24576 16.1 against 17.9.  Below 40
         // blocks this kernel's fp32 sums are no closer to 64 bits than that one's
-        // (17408x3072 6.6e-8 against 6.3e-8; at 5120 7.11e-8 against 7.20e-8).
-        if (nb < 40 || cdiv(n_out, 80 * (int64_t)cus) * 64 * cus > n_out) return -1;
-        pick = SHAPE_SUM;
-    } else {
-        return -1;                                             // gemm_dispatch's plan
+        // (17408x3072 6.6e-8 against 6.3e-8; at 5120 7.11e-8 against 7.20e-8).  More
+        // tokens: gemm_dispatch's plan.
+        return -1;
     }
+    if (!mid_takes(W, n_out, n_tok, nb)) return -1;
     return run_mid(W, Xq, Y, n_out, 0, n_tok, nb, pick, st);
 }
 
