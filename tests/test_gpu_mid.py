@@ -100,7 +100,8 @@ def test_mid_scales_at_the_ends(knobs):
 
 
 @pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33), (17408, 5120, 12),
-                                              (6144, 5120, 651), (10240, 5120, 777), (17408, 5120, 400)])
+                                              (6144, 5120, 651), (10240, 5120, 777), (17408, 5120, 400),
+                                              (17408, 5120, 2100)])
 def test_mid_default_dispatch(n_out, n_in, n_tok):
     """Shapes the default rule gives to this kernel, whole or the tokens past the
     large tiles' whole ones, with and without a workspace (the same bytes), on a
