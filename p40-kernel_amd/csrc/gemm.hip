@@ -1394,7 +1394,12 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
     const int small_sel = knob(pq2host::K_GEMM_SMALL, 0);   // 0 streamed, 1 previous kernel
     if (off32 && n_tok <= 16 && small_sel == 0 && nb % 2 == 0 && nb >= 8 && ((uintptr_t)W & 3u) == 0 &&
         ((uintptr_t)Xq & 15u) == 0) {
-        switch (knob(pq2host::K_GEMM_SMALL_CFG, 0)) {
+        // (BONSAI_GEMM_SMALL_CFG forces a shape, for tests; one that splits K over
+        // more waves than a row has pieces is not taken: its waves without a piece
+        // would fetch the one before the row)
+        const int small_cfg = knob(pq2host::K_GEMM_SMALL_CFG, 0);
+        const int small_ks = small_cfg == 8 ? 16 : small_cfg == 7 || small_cfg == 9 ? 8 : 4;
+        switch (nb / 2 >= small_ks ? small_cfg : 0) {
             case 1: return launch_small_nt<1, 4>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             case 2: return launch_small_nt<2, 4>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             case 3: return launch_small_nt<4, 4>(w, x, Y, (int)n_out, (int)n_tok, nb, st);

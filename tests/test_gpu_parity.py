@@ -1270,3 +1270,24 @@ def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok):
         y = torch.full((n_out,), float("nan"), dtype=torch.float32, device="cuda")
         B.gemv(Wd, dev(xt), y, n_out, n_in)
         assert normwise(got[:, t], host(y)) <= 2 * TOL
+
+
+@pytest.mark.parametrize("n_in,cfg", [(1024, 7), (1024, 8), (1024, 9), (2048, 8), (3840, 8)])
+def test_gemm_forced_wave_split_on_short_rows(n_in, cfg, knobs):
+    """BONSAI_GEMM_SMALL_CFG shapes that split K over 8 or 16 waves, on rows with
+    fewer pieces of two blocks than that: the shape is not taken, the default one
+    runs (the same bytes)."""
+    n_out, n_tok = 50, 9
+    assert n_in // 256 < (16 if cfg == 8 else 8)
+    case(f"gemm {n_out}x{n_in}x{n_tok}, BONSAI_GEMM_SMALL_CFG={cfg} past the row's pieces")
+    W = O.gen_weights(1900 + n_in, n_out, n_in)
+    Xq = O.quantize_chunk_major(O.gen_normal(1901 + n_in, n_tok * n_in).reshape(n_tok, n_in))
+    Wd, Xd = dev(W), dev(Xq)
+    got = []
+    for value in (0, cfg):
+        knobs.set("BONSAI_GEMM_SMALL_CFG", value)
+        Y = torch.full((n_out, n_tok), float("nan"), dtype=torch.float32, device="cuda")
+        B.gemm(Wd, Xd, Y, n_out, n_in, n_tok)
+        got.append(host(Y))
+    np.testing.assert_array_equal(bits(got[1]), bits(got[0]))
+    assert normwise(got[0], O.gemm(W, Xq, n_out, n_in, n_tok, nthreads=16)) <= TOL
