@@ -1439,12 +1439,15 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
         int mi = 8;
         int64_t cols = n_tok;                                   // tokens of the large tiles; the rest on small ones
         int64_t rows = wide != 0 ? pq2::gemm_wide_rows(W, Xq, n_out, n_tok, nb, cus, wide == 2, &mi) : 0;
-        // (BONSAI_GEMM_WIDE other than 1 compares the large tiles, which add in one
-        // order; BONSAI_GEMM_MID forces a small one)
+        // (BONSAI_GEMM_WIDE other than 1, or a knob of the 128-row kernel, compares the
+        // large tiles, which add in one order: they take every token; BONSAI_GEMM_MID
+        // forces a small one)
+        const auto unset = [](pq2host::Knob k) { return knob(k, pq2host::KNOB_UNSET) == pq2host::KNOB_UNSET; };
         if (knob(pq2host::K_GEMM_MID, -1) > 0) {
             const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, cus, st);
             if (rc >= 0) return rc;
-        } else if (wide == 1) {
+        } else if (wide == 1 && unset(pq2host::K_GEMM_F16_BN) && unset(pq2host::K_GEMM_F16_SPLIT) &&
+                   unset(pq2host::K_GEMM_F16_WAVES)) {
             prefill_plan(W, Xq, n_out, n_tok, nb, cus, &cols, &rows, &mi);
         }
         int rc = 0;

@@ -138,3 +138,25 @@ def test_mid_stored_sum_up_to_16_tokens(knobs):
     for knob in (7, 0):
         knobs.set("BONSAI_GEMM_MID", knob)
         assert normwise(gemm(Wd, Xd, n_out, n_in, n_tok), ref) <= TOL
+
+
+@pytest.mark.parametrize("n_out,n_in,n_tok", [(1000, 5120, 17), (1000, 5120, 200), (300, 6144, 77), (129, 1024, 130),
+                                              (200, 2048, 64), (10240, 5120, 777)])
+def test_f16_knobs_reach_the_128_row_kernel(n_out, n_in, n_tok, knobs):
+    """Sizes that the default rule gives to the small tiles, wholly or in part:
+    with a knob of the 128-row kernel set (its token tile, split and waves) that
+    kernel runs, every token of it: the bytes of BONSAI_GEMM_WIDE=0, which are
+    others than the small tiles' (another order of the sums)."""
+    case(f"gemm {n_out}x{n_in}x{n_tok}, the 128-row kernel's knobs")
+    W = O.gen_weights(6600 + n_out, n_out, n_in)
+    Xq = O.quantize_chunk_major(O.gen_normal(6601 + n_tok, n_tok * n_in).reshape(n_tok, n_in))
+    Wd, Xd = dev(W), dev(Xq)
+    knobs.set("BONSAI_GEMM_WIDE", 0)
+    large = gemm(Wd, Xd, n_out, n_in, n_tok)
+    knobs.unset("BONSAI_GEMM_WIDE")
+    assert np.any(large != gemm(Wd, Xd, n_out, n_in, n_tok))
+    for name, value in (("BN", 64), ("BN", 128), ("SPLIT", 0), ("SPLIT", 1), ("WAVES", 8), ("WAVES", 16)):
+        knobs.set("BONSAI_GEMM_F16_" + name, value)
+        np.testing.assert_array_equal(gemm(Wd, Xd, n_out, n_in, n_tok).view(np.uint32), large.view(np.uint32),
+                                      err_msg=f"{name} = {value}")
+        knobs.unset("BONSAI_GEMM_F16_" + name)
