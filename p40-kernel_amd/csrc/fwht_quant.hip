@@ -24,6 +24,7 @@
 
 #include "fwht_device.h"
 #include "host_state.h"
+#include "launch_rules.h"
 #include "../../include/bonsai_p40.h"
 
 using namespace pq2;
@@ -329,11 +330,7 @@ int bonsai_p40_rmsnorm_fwht_quant(const float * x, const float * w, const float 
     const int nw = keep == 1 ? nhb : keep == 2 ? (nhb + 1) / 2 : 16;
     const bool vec = al16(x) && al16(w) && al16(signs);
     hipStream_t st = (hipStream_t)stream;
-    // few tokens: a workgroup per block (spread over the CUs); many: one per
-    // token (each token row read once).  Measured on MI355X (us, per block /
-    // per token): 32 x 5120 4.0 / 4.6, 64 x 5120 4.5 / 4.5, 130 x 5120 5.8 /
-    // 4.6, 512 x 5120 12.1 / 6.7, 40 x 17408 7.9 / 7.3, 100 x 17408 13.0 / 7.6
-    const bool per_block = n_tok * (n / HBLK) <= 256;
+    const bool per_block = pq2::rms_per_block(n_tok, nhb, pq2host::device_info().cus);
 #define PQ2_RMS_LAUNCH(V, S)                                                                        \
     if (per_block)                                                                                  \
         hipLaunchKernelGGL((rms_rot_quant_block_kernel<V, S>), dim3((unsigned)(n / HBLK), (unsigned)n_tok), \

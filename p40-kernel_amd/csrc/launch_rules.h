@@ -1,0 +1,32 @@
+// launch_rules.h -- rules that choose a kernel or a shape from sizes alone:
+// plain host C++, so that they are tested without a GPU.
+#ifndef PQ2_LAUNCH_RULES_H
+#define PQ2_LAUNCH_RULES_H
+
+#include <stdint.h>
+
+namespace pq2 {
+
+// RMSNorm -> FWHT -> Q8_1 of n_tok rows of nhb blocks of 1024: a workgroup per
+// block, which reads its whole row for the sum of squares (true), or one per
+// token, which reads the row once where its waves hold it (up to 32 blocks) and
+// else twice.  The first spreads few tokens over the CUs and its repeated reads
+// cost more with every further round of workgroups; the second takes about as
+// long for one token as for one on each CU, the longer the more blocks a wave
+// has.  So the line is a number of workgroups per block and CU that grows with
+// the row.  Measured on MI355X (256 CUs, us, per block / per token):
+//   up to 14 blocks, 1 a CU: 52 x 5120 5.11 / 4.84, 33 x 8192 5.35 / 4.75
+//   15 to 17, 2: 24 x 15360 6.68 / 6.69, 40 x 16384 7.70 / 6.94, 16 x 17408 6.84 /
+//     7.39, 28 x 17408 7.28 / 7.71, 32 x 17408 7.98 / 7.77
+//   18 and more, 3: 15 x 18432 6.88 / 8.75, 36 x 18432 8.15 / 9.12, 30 x 24576 9.02 /
+//     9.55, 24 x 32768 10.8 / 11.7, 28 x 32768 13.0 / 11.7, 12 x 65536 17.2 / 19.4,
+//     14 x 65536 21.0 / 19.4, 6 x 131072 29.8 / 36.2
+//   256 and more, 4: 4 x 262144 69.5 / 69.7, 1 x 1048576 263 / 271, 2 x 1048576 539 / 271
+inline bool rms_per_block(int64_t n_tok, int64_t nhb, int64_t cus) {
+    const int64_t per_cu = nhb < 15 ? 1 : nhb < 18 ? 2 : nhb < 256 ? 3 : 4;
+    return n_tok <= per_cu * cus && n_tok * nhb <= per_cu * cus;
+}
+
+}  // namespace pq2
+
+#endif

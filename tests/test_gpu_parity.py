@@ -1226,7 +1226,8 @@ def test_unit_dma_probe_runs(n_out, n_in):
 
 
 @pytest.mark.parametrize("n,n_tok", [(1024, 257), (5120, 51), (5120, 52), (16384, 17), (17408, 16), (17408, 301),
-                                     (32768, 9), (33792, 9)])
+                                     (32768, 9), (33792, 9), (16384, 33), (17408, 31), (18432, 43), (32768, 25),
+                                     (33792, 24)])
 def test_rms_prepass_tokens_equal_single_rows(n, n_tok):
     """The many-token kernel (one block, two blocks or more per wave, token
     counts that do not divide by 8, either side of the choice between the two

@@ -1,0 +1,30 @@
+"""CPU: the rules that choose a kernel from sizes alone (csrc/launch_rules.h),
+compiled with g++, on both sides of their lines for a card of 256 CUs."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CUS = 256
+I64 = ctypes.c_int64
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rules") / "rules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "host", "launch_rules.cpp"), "-o", so], check=True)
+    return ctypes.CDLL(so)
+
+
+# (tokens, columns): sizes timed on both kernels, and which was the faster
+@pytest.mark.parametrize("n_tok,n,per_block", [
+    (1, 5120, 1), (51, 5120, 1), (52, 5120, 0), (33, 8192, 0), (2048, 5120, 0), (257, 1024, 0),
+    (16, 17408, 1), (28, 17408, 1), (32, 17408, 0), (48, 17408, 0),
+    (15, 18432, 1), (36, 18432, 1), (30, 24576, 1), (24, 32768, 1), (28, 32768, 0), (20, 33792, 1), (24, 33792, 0),
+    (12, 65536, 1), (14, 65536, 0), (6, 131072, 1), (3, 262144, 1), (1, 1048576, 1), (2, 1048576, 0), (1, 2097152, 0),
+    ((1 << 31) - 1, 1024, 0), ((1 << 31) - 1, (1 << 31) - 1024, 0)])
+def test_rms_prepass_kernel(rules, n_tok, n, per_block):
+    assert rules.rms_per_block(I64(n_tok), I64(n // 1024), I64(CUS)) == per_block
