@@ -26,6 +26,7 @@
 // * Small batches (n_tok <= 32) use a 128 x 32 tile (4 waves stacked on rows).
 #include "pq2_device.h"
 #include "host_state.h"
+#include "launch_rules.h"
 #include "../../include/bonsai_p40.h"
 
 #include <stdlib.h>
@@ -1411,19 +1412,12 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
             case 8: return launch_small_nt<1, 16>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             default: break;
         }
-        // measured on MI355X: 16-row workgroups; K split 8 ways up to 8 tokens
-        // (more waves in flight), 4 ways for 9..16 tokens (the ring's LDS)
+        // measured on MI355X: 16-row workgroups, K split 8 ways up to 8 tokens
+        // (more waves in flight); past that see the rule
         if (n_tok <= 8 && nb >= 16) return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
-        // 9..16 tokens in one round of CUs: K split 8 ways all the same, on 16 rows
-        // or on 32.  The ring then fills a CU, so past one round 4 ways stay.  Us,
-        // 16 rows / 4 ways -> this: 1024x5120 with 12 tokens 5.8 -> 5.2, 4096x17408
-        // 15.7 -> 11.5 (16 rows); 6144x5120 7.7 -> 7.4, 5120x6144 8.4 -> 7.4,
-        // 5120x17408 19.3 -> 17.5 (32 rows); 10240x5120 stays (9.3 against 13.2).
-        // Below 40 blocks 8 partial sums are no closer to 64 bits than 4
-        // (1024x2048 6.4e-8 against 5.7e-8; at 5120 columns 7.1e-8 against 7.4e-8).
-        const int64_t cus = gemm_cu_count();
-        if (nb >= 40 && n_out <= 16 * cus) return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
-        if (nb >= 40 && n_out <= 32 * cus) return launch_small_nt<2, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
+        const pq2::SmallShape shape = pq2::small_shape(n_out, nb, gemm_cu_count());
+        if (shape.rt == 2) return launch_small_nt<2, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
+        if (shape.ks == 8) return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
         return launch_small_nt<1, 4>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
     }
     if (n_tok <= 16 && nb % 8 == 0 && ((uintptr_t)W & 3u) == 0 && skinny_lds <= (size_t)skinny_lds_limit()) {

@@ -27,6 +27,28 @@ inline bool rms_per_block(int64_t n_tok, int64_t nhb, int64_t cus) {
     return n_tok <= per_cu * cus && n_tok * nhb <= per_cu * cus;
 }
 
+// Rows (16 rt) and waves over K (ks) of a workgroup of the streamed kernel for 9
+// to 16 tokens.  8 ways over K keep more loads in flight than 4, but their ring
+// fills a CU where two 4-way ones fit, so they pay in one round of CUs only, on
+// 16 rows or else on 32.  Measured on MI355X (256 CUs, us, 9 / 12 / 16 tokens, 16
+// rows and 4 ways -> this): 16 rows, 1024x5120 5.9 6.0 6.2 -> 5.5 5.5 5.6, 4096x17408
+// 15.8 16.0 16.4 -> 12.2 12.4 12.8; 32 rows, 5120x6144 8.9 8.9 9.0 -> 8.0 8.0 8.4,
+// 5120x17408 18.6 18.6 18.8 -> 16.5 16.6 17.2, 8192x8192 11.2 11.4 11.6 -> 10.7 10.6
+// 10.9.  On 40 to 47 blocks the 32-row gain is small (6144x5120 2 %) and gone at
+// either end (4097x5120 7.5 -> 7.6..7.8, 8192x5120 8.4 -> 8.5), so the range stops
+// short of both there.  Below 40 blocks 8 partial sums are further from 64 bits than
+// 4, from 40 on no further (4 / 8 ways, 1e-8: 2048 columns 5.7 / 6.4, 3072 6.2 /
+// 6.6, 4096 6.75 / 6.88, 5120 7.20 / 7.13, 6144 7.65 / 7.35, 17408 11.4 / 9.5).
+struct SmallShape {
+    int rt, ks;
+};
+inline SmallShape small_shape(int64_t n_out, int nb, int64_t cus) {
+    if (nb < 40) return {1, 4};
+    if (n_out <= 16 * cus) return {1, 8};
+    if (nb < 48 ? 2 * n_out > 33 * cus && n_out <= 28 * cus : n_out <= 32 * cus) return {2, 8};
+    return {1, 4};
+}
+
 }  // namespace pq2
 
 #endif

@@ -3,4 +3,8 @@
 
 extern "C" {
 int rms_per_block(int64_t n_tok, int64_t nhb, int64_t cus) { return pq2::rms_per_block(n_tok, nhb, cus); }
+int small_shape(int64_t n_out, int nb, int64_t cus) {
+    const pq2::SmallShape s = pq2::small_shape(n_out, nb, cus);
+    return 16 * s.rt * 100 + s.ks;
+}
 }

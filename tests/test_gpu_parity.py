@@ -1245,14 +1245,20 @@ def test_rms_prepass_tokens_equal_single_rows(n, n_tok):
     np.testing.assert_array_equal(host(got).reshape(n // 32, n_tok, 36), np.stack(rows, axis=1))
 
 
-@pytest.mark.parametrize("n_out,n_in,n_tok", [(19, 17408, 9), (1024, 5120, 12), (4096, 5120, 13), (4097, 6144, 16),
-                                              (8191, 5120, 12), (8193, 5120, 10), (5120, 4992, 12)])
-def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok):
+# the last figure is the BONSAI_GEMM_SMALL_CFG that the default shape equals in
+# its bytes: 1 for K split 4 ways, 7 for 8 ways (on 16 rows or 32), 0 where the
+# block count is odd and another kernel runs
+@pytest.mark.parametrize("n_out,n_in,n_tok,cfg", [
+    (19, 17408, 9, 7), (1024, 5120, 12, 7), (4096, 5120, 13, 7), (4097, 6144, 16, 7), (8191, 6144, 12, 7),
+    (8193, 5120, 10, 1), (5120, 4992, 12, 0), (5120, 4864, 12, 1), (4097, 5120, 12, 1), (4225, 5120, 16, 7), (7168, 5120, 9, 7),
+    (7169, 5120, 13, 1)])
+def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok, cfg, knobs):
     """9..16 tokens on the streamed kernel at the edges of its workgroup shapes
     (16 rows with K split 8 ways, 32 rows past one round of those, 16 rows with
     K split 4 ways past one round of these and on short rows) and of its rings
     (12 and 16 tokens): against the oracle on the first, middle and last rows,
-    and against one GEMV per token."""
+    against one GEMV per token, and the bytes of the K split that the size
+    takes, which are not those of the other."""
     case(f"gemm streamed {n_out}x{n_in}x{n_tok}")
     W = O.gen_weights(1800 + n_out + n_tok, n_out, n_in)
     Xq = O.quantize_chunk_major(O.gen_normal(1801 + n_in, n_tok * n_in).reshape(n_tok, n_in))
@@ -1271,6 +1277,10 @@ def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok):
         y = torch.full((n_out,), float("nan"), dtype=torch.float32, device="cuda")
         B.gemv(Wd, dev(xt), y, n_out, n_in)
         assert normwise(got[:, t], host(y)) <= 2 * TOL
+    for value in (1, 7):
+        knobs.set("BONSAI_GEMM_SMALL_CFG", value)
+        B.gemm(Wd, dev(Xq), Y, n_out, n_in, n_tok)
+        assert np.array_equal(bits(host(Y)), bits(got)) == (cfg in (0, value)), value
 
 
 @pytest.mark.parametrize("n_in,cfg", [(1024, 7), (1024, 8), (1024, 9), (2048, 8), (3840, 8)])

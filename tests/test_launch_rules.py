@@ -28,3 +28,13 @@ def rules(tmp_path_factory):
     ((1 << 31) - 1, 1024, 0), ((1 << 31) - 1, (1 << 31) - 1024, 0)])
 def test_rms_prepass_kernel(rules, n_tok, n, per_block):
     assert rules.rms_per_block(I64(n_tok), I64(n // 1024), I64(CUS)) == per_block
+
+
+# rows of a workgroup and waves over K of the streamed kernel for 9 to 16 tokens
+@pytest.mark.parametrize("n_out,n_in,rows,waves", [
+    (1, 5120, 16, 8), (4096, 5120, 16, 8), (4097, 5120, 16, 4), (4224, 5120, 16, 4), (4225, 5120, 32, 8),
+    (7168, 5120, 32, 8), (7169, 5120, 16, 4), (8192, 5120, 16, 4), (10240, 5120, 16, 4),
+    (4096, 6144, 16, 8), (4097, 6144, 32, 8), (8192, 6144, 32, 8), (8193, 6144, 16, 4), (5120, 17408, 32, 8),
+    (1024, 4992, 16, 4), (8192, 4096, 16, 4), ((1 << 31) - 1, 5120, 16, 4)])
+def test_streamed_shape_9_to_16_tokens(rules, n_out, n_in, rows, waves):
+    assert rules.small_shape(I64(n_out), n_in // 128, I64(CUS)) == 100 * rows + waves
