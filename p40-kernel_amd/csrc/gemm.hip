@@ -628,15 +628,21 @@ int launch_small_t(const uint8_t * W, const uint8_t * X, float * Y, int n_out, i
     return (int)hipGetLastError();
 }
 
+// The ring holds 2, 4, 8 or 16 tokens; the shapes that small_shape picks for 9 to
+// 16 have one of 12 too: 4 instead of 5 DMA instructions of activation a piece
+// (17408-column rows, 12 tokens, 19.5 -> 18.8 us; 10240x5120 9.6 -> 9.3).  32 rows
+// and 8 waves run 9 tokens and more only.
 template <int RT, int KS>
 int launch_small_nt(const uint8_t * W, const uint8_t * X, float * Y, int n_out, int n_tok, int nb,
                     hipStream_t st) {
-    if (n_tok <= 2) return launch_small_t<RT, KS, 2>(W, X, Y, n_out, n_tok, nb, st);
-    if (n_tok <= 4) return launch_small_t<RT, KS, 4>(W, X, Y, n_out, n_tok, nb, st);
-    if (n_tok <= 8) return launch_small_t<RT, KS, 8>(W, X, Y, n_out, n_tok, nb, st);
-    // a ring sized for 12 tokens is 4 instead of 5 DMA instructions of activation
-    // a piece (17408-column rows, 12 tokens, 19.5 -> 18.8 us; 10240x5120 9.6 -> 9.3)
-    if (n_tok <= 12) return launch_small_t<RT, KS, 12>(W, X, Y, n_out, n_tok, nb, st);
+    constexpr bool tall = RT == 2 && KS == 8, picked = tall || (RT == 1 && (KS == 4 || KS == 8));
+    if constexpr (!tall) {
+        if (n_tok <= 2) return launch_small_t<RT, KS, 2>(W, X, Y, n_out, n_tok, nb, st);
+        if (n_tok <= 4) return launch_small_t<RT, KS, 4>(W, X, Y, n_out, n_tok, nb, st);
+        if (n_tok <= 8) return launch_small_t<RT, KS, 8>(W, X, Y, n_out, n_tok, nb, st);
+    }
+    if constexpr (picked)
+        if (n_tok <= 12) return launch_small_t<RT, KS, 12>(W, X, Y, n_out, n_tok, nb, st);
     return launch_small_t<RT, KS, 16>(W, X, Y, n_out, n_tok, nb, st);
 }
 
@@ -1408,8 +1414,10 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
             case 5: return launch_small_nt<2, 2>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             case 6: return launch_small_nt<4, 2>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             case 7: return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
-            case 9: return launch_small_nt<2, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
             case 8: return launch_small_nt<1, 16>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
+            case 9:
+                if (n_tok > 8) return launch_small_nt<2, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
+                break;
             default: break;
         }
         // measured on MI355X: 16-row workgroups, K split 8 ways up to 8 tokens

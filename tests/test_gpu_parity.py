@@ -1277,10 +1277,11 @@ def test_gemm_streamed_9_to_16_tokens(n_out, n_in, n_tok, cfg, knobs):
         y = torch.full((n_out,), float("nan"), dtype=torch.float32, device="cuda")
         B.gemv(Wd, dev(xt), y, n_out, n_in)
         assert normwise(got[:, t], host(y)) <= 2 * TOL
-    for value in (1, 7):
+    for value in (1, 7, 9):                                   # 9: 8 ways on 32 rows
         knobs.set("BONSAI_GEMM_SMALL_CFG", value)
+        Y.fill_(float("nan"))
         B.gemm(Wd, dev(Xq), Y, n_out, n_in, n_tok)
-        assert np.array_equal(bits(host(Y)), bits(got)) == (cfg in (0, value)), value
+        assert np.array_equal(bits(host(Y)), bits(got)) == (cfg == 0 or (cfg == 7) == (value > 1)), value
 
 
 @pytest.mark.parametrize("n_in,cfg", [(1024, 7), (1024, 8), (1024, 9), (2048, 8), (3840, 8)])

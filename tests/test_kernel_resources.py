@@ -28,7 +28,7 @@ def rows():
 def test_every_kernel_family_is_present(rows):
     fams = {kr.family(r) for r in rows}
     for f in ("gemv_nb_kernel", "gemv_stream_kernel", "gemm_wide_kernel", "gemm_f16_kernel", "gemm_bd_kernel",
-              "gemm_small_kernel", "rot_quant_kernel", "rms_rot_quant_kernel", "swiglu_rot_quant_kernel",
+              "gemm_mid_kernel", "gemm_small_kernel", "rot_quant_kernel", "rms_rot_quant_kernel", "swiglu_rot_quant_kernel",
               "quant_kernel", "repack_kernel", "chain_kernel"):
         assert f in fams, f
 
@@ -75,3 +75,15 @@ def test_wide_prefill_kernel_keeps_two_waves_per_simd(rows):
     for r in wide:
         assert r["max_wg"] == 512
         assert r["vgpr"] + r["agpr"] <= 256, (r["name"], r["vgpr"], r["agpr"])
+
+
+def test_streamed_kernel_is_built_for_the_shapes_in_use(rows):
+    # rings of 2, 4, 8 and 16 tokens for the eight shapes that BONSAI_GEMM_SMALL_CFG
+    # can force; the three that 9 to 16 tokens pick from have one of 12 too, and the
+    # third of them (32 rows, 8 waves) no ring of fewer
+    import re
+    built = sorted(tuple(int(v) for v in re.search(r"gemm_small_kernel<(\d+), ?(\d+), ?(\d+)>", r["name"]).groups())
+                   for r in rows if kr.family(r) == "gemm_small_kernel")
+    shapes = [(1, 4), (2, 4), (4, 4), (1, 2), (2, 2), (4, 2), (1, 8), (1, 16)]
+    assert built == sorted([(rt, ks, nt) for rt, ks in shapes for nt in (2, 4, 8, 16)] +
+                           [(1, 4, 12), (1, 8, 12), (2, 8, 12), (2, 8, 16)])
