@@ -32,10 +32,10 @@
 
 #include "pq2_device.h"
 #include "host_state.h"
+#include "launch_rules.h"
 #include "../../include/bonsai_p40.h"
 
 #include <stdint.h>
-#include <algorithm>
 
 using namespace pq2;
 
@@ -301,35 +301,6 @@ int launch_mid(const uint8_t * w, const uint8_t * x, float * Y, int64_t n_out, i
     return (int)hipGetLastError();
 }
 
-// Tile shapes, and per shape the time of one step on one CU (MI355X, us, the
-// slope over K of one round of workgroups); a CU holds one workgroup, a launch
-// starts and reduces in about 4 us, and many full rounds lower the clock
-// (17408x5120 with 400 tokens: 8 rounds of 80 x 48 in 171 us, 33 tokens: one in 22).  80 x 16 tiles that read the stored
-// sums run batches of up to 16 tokens only.
-struct Shape {
-    int mi, ni;
-    float us;
-    bool sum;
-};
-constexpr int SHAPES = 9, SHAPE_SUM = 6;
-constexpr Shape shapes[SHAPES] = {{5, 3, 3.6f, false},  {3, 2, 1.8f, false}, {5, 2, 2.5f, false},
-                                  {4, 2, 2.05f, false}, {4, 3, 2.8f, false}, {2, 2, 1.45f, false},
-                                  {5, 1, 1.9f, true},   {5, 1, 1.8f, false}, {3, 1, 1.2f, false}};
-
-// The fastest shape for n_tok tokens, and its time (mid_takes first: 32-bit
-// arithmetic, this runs on every call)
-int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus, float * us) {
-    int pick = -1;
-    for (int k = 0; k < SHAPES; ++k) {
-        if (shapes[k].sum) continue;
-        const uint32_t bm = 16 * shapes[k].mi, bn = 16 * shapes[k].ni;
-        const uint32_t wgs = (((uint32_t)n_out + bm - 1) / bm) * (((uint32_t)n_tok + bn - 1) / bn);
-        const float r = (float)((wgs + (uint32_t)cus - 1) / (uint32_t)cus), t = 4.0f + r * (1.0f + 0.02f * std::min(r, 8.0f)) * (float)(nb / 8) * shapes[k].us;
-        if (pick < 0 || t < *us) *us = t, pick = k;
-    }
-    return pick;
-}
-
 // Whole steps of 8 blocks, 16-byte DMA of W's rows, 32-bit offsets (80 rows of
 // W, a block's 4 chunks of X), a grid of under 2^32 threads
 bool mid_takes(const void * W, int64_t n_out, int64_t n_tok, int nb) {
@@ -347,7 +318,7 @@ int run_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t f
         case 3: return launch_mid<4, 2>(w, x, Y, n_out, first, n_tok, nb, st);
         case 4: return launch_mid<4, 3>(w, x, Y, n_out, first, n_tok, nb, st);
         case 5: return launch_mid<2, 2>(w, x, Y, n_out, first, n_tok, nb, st);
-        case SHAPE_SUM: return launch_mid<5, 1, true>(w, x, Y, n_out, first, n_tok, nb, st);
+        case MID_SUM: return launch_mid<5, 1, true>(w, x, Y, n_out, first, n_tok, nb, st);
         case 7: return launch_mid<5, 1>(w, x, Y, n_out, first, n_tok, nb, st);
         default: return launch_mid<3, 1>(w, x, Y, n_out, first, n_tok, nb, st);
     }
@@ -362,20 +333,25 @@ namespace pq2 {
 // shape, whatever the tokens (tests).
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st) {
     const int forced = pq2host::knob(pq2host::K_GEMM_MID, -1);
-    int pick = SHAPE_SUM;
+    int pick = MID_SUM;
     if (forced > 0) {
-        pick = (forced < SHAPES ? forced : SHAPES) - 1;
+        pick = (forced < MID_SHAPES ? forced : MID_SHAPES) - 1;
     } else if (forced == 0 || n_tok > 16 || nb < 40 || n_out <= 64 * (int64_t)cus ||
                cdiv(n_out, 80 * (int64_t)cus) * 64 * cus > n_out) {
-        // 9 to 16 tokens: the streamed kernel (gemm_small_kernel) takes 64 rows a CU
-        // and round, 80 x 16 tiles here 80 in the same time, so they are the faster
-        // where their rounds, rounded up, are no more than that one's as a fraction.
-        // Measured (us, streamed -> here, 12 tokens, n_in 5120): 17408 rows 15.5 ->
-        // 13.4, 49152 29.4 -> 28.1, 248320 144 -> 118, 16385x17408 38.1 -> 35.4; on the
-        // other side 10240 rows 9.6 against 10.2, 24576 16.1 against 17.9.  Below 40
-        // blocks this kernel's fp32 sums are no closer to 64 bits than that one's
-        // (17408x3072 6.6e-8 against 6.3e-8; at 5120 7.11e-8 against 7.20e-8).  More
-        // tokens: gemm_dispatch's plan.
+        // 9 to 16 tokens on tall matrices.  The streamed kernel (gemm_small_kernel)
+        // costs by the rows, about one unit for each 64 of a CU; the tiles here by
+        // whole multiples of 80 rows a CU, each about that unit too (two workgroups
+        // share a CU, the second adds what a further round would).  So the tiles are
+        // taken where their multiples, rounded up, are no more than those units as a
+        // fraction, past the first.  Measured on MI355X (256 CUs, us, streamed /
+        // tiles, 9, 12, 16 tokens): 17408x5120 13.6 13.8 14.5 / 13.2 13.2 13.3, 20481
+        // rows 14.9 14.8 15.8 / 18.1 18.1 18.0, 28000 19.5 19.9 21.4 / 19.8 19.8 20.1, 32768
+        // 22.0 22.4 24.0 / 20.6 20.2 20.3, 40961 25.2 25.9 27.7 / 27.7 28.3 28.2, 49152
+        // 28.4 28.4 30.4 / 28.8 28.8 29.1, 57344 34.6 35.7 38.7 / 30.3 30.3 30.1; 17408x8192
+        // 21.2 21.8 23.8 / 19.8 19.8 19.8, 24576x8192 23.5 23.9 25.4 / 27.7 27.6 27.9.
+        // Below 40 blocks 8 partial sums are further from 64 bits than that kernel's
+        // 4 (3072 columns 6.6e-8 against 6.2e-8; at 5120 7.1e-8 against 7.2e-8).
+        // More tokens: gemm_dispatch's plan.
         return -1;
     }
     if (!mid_takes(W, n_out, n_tok, nb)) return -1;

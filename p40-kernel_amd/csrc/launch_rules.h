@@ -49,6 +49,47 @@ inline SmallShape small_shape(int64_t n_out, int nb, int64_t cus) {
     return {1, 4};
 }
 
+// Tile shapes of the small-tile GEMM (gemm_mid.hip): 16 mi rows x 16 ni tokens
+// (sum: the stored sums are read, batches of up to 16 tokens only), and the time
+// of one step of 8 blocks on one CU (MI355X, us, the slope over K of one round of
+// workgroups).  A CU holds one workgroup of the wider tiles, whose registers or
+// LDS leave no room for a second.  Of the 16-token tiles it holds two (116 and 95
+// VGPRs, 72 and 52 KB of LDS): us2 is a step of both, so a second one costs about
+// 0.6 of a round.  Measured (us, 5120 columns, 256 / 257 / 512 / 513 workgroups): 80 x 32
+// 18.7 32.0 35.9 48.8, 80 x 16 13.7 18.1 20.9 28.2, 48 x 16 10.2 13.3 14.6 19.3.
+struct MidShape {
+    int mi, ni;
+    float us, us2;
+    bool sum;
+};
+constexpr int MID_SHAPES = 9, MID_SUM = 6;
+constexpr MidShape mid_shapes[MID_SHAPES] = {
+    {5, 3, 3.6f, 0.0f, false},  {3, 2, 1.8f, 0.0f, false},  {5, 2, 2.5f, 0.0f, false},
+    {4, 2, 2.05f, 0.0f, false}, {4, 3, 2.8f, 0.0f, false},  {2, 2, 1.45f, 0.0f, false},
+    {5, 1, 1.9f, 3.0f, true},   {5, 1, 1.8f, 2.85f, false}, {3, 1, 1.2f, 1.98f, false}};
+
+// The fastest shape for n_tok tokens of rows of nb blocks, and its estimated time:
+// rounds of workgroups, 4 us to start and reduce, and a clock that many full
+// rounds lower (17408x5120 with 400 tokens: 8 rounds of 80 x 48 in 171 us, 33
+// tokens: one in 22).  32-bit arithmetic, this runs on every call: the caller has
+// seen that there are under 2^22 tiles of 32 x 16.
+inline int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus, float * us) {
+    int pick = -1;
+    const uint32_t c = (uint32_t)cus;
+    for (int k = 0; k < MID_SHAPES; ++k) {
+        const MidShape & s = mid_shapes[k];
+        if (s.sum) continue;
+        const uint32_t bm = 16 * s.mi, bn = 16 * s.ni;
+        const uint32_t wgs = (((uint32_t)n_out + bm - 1) / bm) * (((uint32_t)n_tok + bn - 1) / bn);
+        const uint32_t rounds = (wgs + c - 1) / c;
+        const float r = (float)rounds;
+        const float step = s.us2 == 0.0f ? r * s.us : (float)(rounds / 2) * s.us2 + (float)(rounds % 2) * s.us;
+        const float t = 4.0f + (1.0f + 0.02f * (r < 8.0f ? r : 8.0f)) * (float)(nb / 8) * step;
+        if (pick < 0 || t < *us) *us = t, pick = k;
+    }
+    return pick;
+}
+
 }  // namespace pq2
 
 #endif

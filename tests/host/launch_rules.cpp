@@ -7,4 +7,14 @@ int small_shape(int64_t n_out, int nb, int64_t cus) {
     const pq2::SmallShape s = pq2::small_shape(n_out, nb, cus);
     return 16 * s.rt * 100 + s.ks;
 }
+int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus) {
+    float us = 0.0f;
+    const pq2::MidShape & s = pq2::mid_shapes[pq2::mid_pick(n_out, n_tok, nb, cus, &us)];
+    return 16 * s.mi * 1000 + 16 * s.ni;
+}
+float mid_us(int64_t n_out, int64_t n_tok, int nb, int cus) {
+    float us = 0.0f;
+    pq2::mid_pick(n_out, n_tok, nb, cus, &us);
+    return us;
+}
 }

@@ -38,3 +38,16 @@ def test_rms_prepass_kernel(rules, n_tok, n, per_block):
     (1024, 4992, 16, 4), (8192, 4096, 16, 4), ((1 << 31) - 1, 5120, 16, 4)])
 def test_streamed_shape_9_to_16_tokens(rules, n_out, n_in, rows, waves):
     assert rules.small_shape(I64(n_out), n_in // 128, I64(CUS)) == 100 * rows + waves
+
+
+# sizes with every shape timed: the pick, and the time measured for it (us), which
+# the estimate has to meet within a quarter
+@pytest.mark.parametrize("n_out,n_in,n_tok,bm,bn,us", [
+    (17408, 5120, 17, 80, 32, 17.4), (17408, 5120, 33, 80, 48, 22.5), (17408, 5120, 100, 80, 16, 47.1),
+    (8703, 5120, 100, 80, 16, 26.5), (2560, 17408, 140, 48, 16, 37.8), (4096, 1024, 80, 48, 16, 5.6),
+    (512, 5120, 64, 48, 16, 9.1), (4096, 1024, 33, 32, 32, 5.0), (6144, 5120, 50, 48, 32, 13.4),
+    (5120, 17408, 80, 64, 32, 39.8), (10240, 5120, 140, 64, 48, 36.3), (6144, 5120, 140, 80, 48, 22.1)])
+def test_small_tile_shape(rules, n_out, n_in, n_tok, bm, bn, us):
+    assert rules.mid_pick(I64(n_out), I64(n_tok), n_in // 128, CUS) == 1000 * bm + bn
+    rules.mid_us.restype = ctypes.c_float
+    assert 0.75 * us < rules.mid_us(I64(n_out), I64(n_tok), n_in // 128, CUS) < 1.25 * us
