@@ -1303,61 +1303,12 @@ int gemm_wide_launch_ws(const void * W, const void * Xq, float * Y, int64_t n_ou
                         int mi, void * ws, hipStream_t st);
 // gemm_mid.hip: small tiles with K split over a workgroup's waves; -1 if not applicable
 int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t n_tok, int nb, int cus, hipStream_t st);
-float gemm_mid_us(const void * W, int64_t n_out, int64_t first, int64_t n_tok, int nb, int cus);
+bool gemm_mid_takes(const void * W, int64_t n_out, int64_t n_tok, int nb);
 int gemm_mid_tail(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb,
                   int cus, hipStream_t st);
 }
 
 namespace {
-
-// Time (us) of tokens [0, cols) on the large tiles, rows as gemm_wide_rows
-// gives them: rounds of workgroups times what a round takes a block of K
-// (MI355X: 4.5 us on 256-row tiles, 3.45 on 160-row ones, 1.42 on 128 x 128,
-// 1.05 on 128 x 64)
-float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows, int mi) {
-    float us = 0.0f;
-    if (rows > 0) us = (mi == 8 ? 4.5f : 3.45f) * (float)cdiv(cdiv(rows, 32 * mi) * cdiv(cols, 256), cus);
-    if (rows < n_out) {
-        // gemm_prefill_f16's choice
-        const int64_t R = cdiv(n_out - rows, GF_BM), T = cdiv(cols, 128), full = R * T / cus, rest = R * T - full * cus;
-        if (2 * R * T <= cus) us += 1.05f;
-        else if (full >= 1 && rest > 0 && 2 * rest <= cus && full * cus % T == 0 && (R - full * cus / T) * cdiv(cols, 64) <= cus)
-            us += 1.42f * (float)full + 1.05f;
-        else us += 1.42f * (float)cdiv(R * T, cus);
-    }
-    return us * (float)nb;
-}
-
-// The tiles of a prefill: tokens [0, cols) on the large ones, the first rows of
-// them on the wide kernel (tile height mi), tokens [cols, n_tok) on the small
-// ones (gemm_mid.hip; cols = 0: all of them).  rows and mi come as
-// gemm_wide_rows gives them for every token; another plan has to be 5 % faster
-// by its estimate.  Small tiles take over the whole product where large ones
-// would leave most CUs idle, or the tokens past the whole large tiles where
-// these would start another round, and rows whose wide tiles are short of a round
-// take 128-row tiles where those have fewer empty tokens.  Measured (us, large
-// tiles as gemm_wide_rows has them -> this plan): 17408x5120 with 20 tokens 57
-// -> 17, 33 54 -> 22, 140 101 -> 63, 400 159 -> 126; 5120x17408 with 100 132 ->
-// 45, 800 361 -> 213; 10240x5120 with 386 102 -> 69, 777 139 -> 132 (768 + 9
-// tokens), 1166 229 -> 180; unchanged 17408x5120 with 1500, 10240x5120 with 1900.
-void prefill_plan(const void * W, const void * Xq, int64_t n_out, int64_t n_tok, int nb, int cus, int64_t * cols,
-                  int64_t * rows, int * mi) {
-    float best = 0.95f * large_us(n_out, n_tok, nb, cus, *rows, *mi);
-    const float small = pq2::gemm_mid_us(W, n_out, 0, n_tok, nb, cus);
-    if (small > 0.0f && small < best) best = small, *cols = 0, *rows = 0;
-    // gemm_wide_rows looks at the tokens that it is given only
-    if ((uint64_t)n_tok * Q81_BYTES * 4ull * (uint64_t)nb >= (1ull << 31)) return;
-    for (int64_t c : {n_tok, n_tok / 128 * 128, n_tok / 256 * 256}) {
-        float us = 0.0f;
-        if (c < n_tok) us = pq2::gemm_mid_us(W, n_out, c, n_tok, nb, cus);
-        if (c == 0 || (c < n_tok && us == 0.0f)) continue;
-        int m = 8;
-        const int64_t r = pq2::gemm_wide_rows(W, Xq, n_out, c, nb, cus, false, &m);
-        const float wide = us + large_us(n_out, c, nb, cus, r, m), plain = us + large_us(n_out, c, nb, cus, 0, 8);
-        if (r > 0 && (c == n_tok || c % 256 == 0) && wide < best) best = wide, *cols = c, *rows = r, *mi = m;
-        if (plain < best) best = plain, *cols = c, *rows = 0;
-    }
-}
 
 // bonsai_p40_gemm's dispatch; ws (non-NULL: large enough and aligned, checked
 // by the caller) lets the long-prompt kernel take the activation by DMA
@@ -1450,7 +1401,8 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
             if (rc >= 0) return rc;
         } else if (wide == 1 && unset(pq2host::K_GEMM_F16_BN) && unset(pq2host::K_GEMM_F16_SPLIT) &&
                    unset(pq2host::K_GEMM_F16_WAVES)) {
-            prefill_plan(W, Xq, n_out, n_tok, nb, cus, &cols, &rows, &mi);
+            const bool aligned = (((uintptr_t)W | (uintptr_t)Xq) & 3u) == 0;
+            pq2::prefill_plan(aligned, pq2::gemm_mid_takes(W, n_out, n_tok, nb), n_out, n_tok, nb, cus, &cols, &rows, &mi);
         }
         int rc = 0;
         if (rows > 0) {

@@ -358,16 +358,13 @@ int gemm_mid(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t 
     return run_mid(W, Xq, Y, n_out, 0, n_tok, nb, pick, st);
 }
 
-// Estimated time (us) of tokens [first, n_tok) here; 0 where the kernel does
-// not take them
-float gemm_mid_us(const void * W, int64_t n_out, int64_t first, int64_t n_tok, int nb, int cus) {
-    float us = 0.0f;
-    if (pq2host::knob(pq2host::K_GEMM_MID, -1) < 0 && mid_takes(W, n_out, n_tok, nb))
-        mid_pick(n_out, n_tok - first, nb, cus, &us);
-    return us;
+// Whether the kernel's requirements hold for more than 16 tokens (and
+// BONSAI_GEMM_MID does not decide)
+bool gemm_mid_takes(const void * W, int64_t n_out, int64_t n_tok, int nb) {
+    return pq2host::knob(pq2host::K_GEMM_MID, -1) < 0 && mid_takes(W, n_out, n_tok, nb);
 }
 
-// Tokens [first, n_tok) of the product (gemm_mid_us takes them)
+// Tokens [first, n_tok) of the product (gemm_mid_takes it)
 int gemm_mid_tail(const void * W, const void * Xq, float * Y, int64_t n_out, int64_t first, int64_t n_tok, int nb,
                   int cus, hipStream_t st) {
     float us = 0.0f;

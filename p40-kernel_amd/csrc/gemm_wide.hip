@@ -58,10 +58,10 @@
 #include "pq2_device.h"
 #include "gemv_device.h"
 #include "host_state.h"
+#include "launch_rules.h"
 #include "../../include/bonsai_p40.h"
 
 #include <stdint.h>
-#include <algorithm>
 #include <type_traits>
 
 using namespace pq2;
@@ -529,43 +529,17 @@ gemm_wide_kernel(const uint8_t * __restrict__ W, const uint8_t * __restrict__ X,
 
 namespace pq2 {
 
-// Rows [0, rows) of the product that the wide kernel takes, and its tile
-// height (*mi = 8: 256 rows, 5: 160 rows): the whole 256-row tiles whose
-// 256 x 256 tiles fill whole rounds of the device's CUs (the caller runs the
-// remaining rows on the 128-row kernel), or, short of one round, every row on
-// 256- or 160-row tiles where one round of them holds at least 3/4 of a full
-// round's outputs; 0 where the kernel's requirements do not hold or its tiles
-// would fill too little of a round.  force: every row whenever the requirements
-// hold (tests; the BONSAI_GEMM_WIDE_MI knob picks the tile height there).
+// Rows [0, rows) of the product that the wide kernel takes, and its tile height
+// (wide_rows of launch_rules.h, where W and Xq are aligned for it).  force: every
+// row whenever the requirements hold (tests; the BONSAI_GEMM_WIDE_MI knob picks
+// the tile height there).
 int64_t gemm_wide_rows(const void * W, const void * Xq, int64_t n_out, int64_t n_tok, int nb, int cus, bool force,
                        int * mi) {
     *mi = 8;
-    if (nb < 2 || nb % 2 != 0 || ((uintptr_t)W & 3u) != 0 || ((uintptr_t)Xq & 3u) != 0) return 0;
-    if ((uint64_t)n_out * PQ2_BYTES * (uint64_t)nb >= (1ull << 31)) return 0;      // buffer ranges are int
-    if ((uint64_t)n_tok * Q81_BYTES * 4ull * (uint64_t)nb >= (1ull << 31)) return 0;
-    if (force) {
-        *mi = pq2host::knob(pq2host::K_GEMM_WIDE_MI, 8) == 5 ? 5 : 8;
-        return n_out;
-    }
-    const int64_t T = (n_tok + WB_N - 1) / WB_N;
-    if (4 * n_tok < 3 * T * WB_N) return 0;                                       // token tiles mostly empty
-    // 256-row tiles over the rows whose tiles fill whole rounds
-    const int64_t R = n_out / 256, rounds = R * T / cus;
-    if (rounds >= 1) return std::min<int64_t>(R, rounds * cus / T) * 256;
-    // Less than one round: a round of wide tiles takes about the same time
-    // however many CUs it fills, so one pays where at least 3/4 of a full
-    // round's outputs are real (measured on MI355X, one process, us, LDS kernel
-    // -> wide: 17408x5120 M = 768 225 -> 181 (256 rows), M = 512 165 -> 138
-    // (160 rows), 6144x5120 M = 2048 189 -> 180 (256 rows); at 5/8 and below
-    // the LDS kernel stays faster: 17408x5120 M = 384 116 against 137,
-    // 5120x6144 M = 1024 126 against 160)
-    const int64_t outputs = n_out * n_tok;
-    if ((n_out + 255) / 256 * T <= cus && 4 * outputs >= 3 * (int64_t)cus * 256 * WB_N) return n_out;
-    if ((n_out + 159) / 160 * T <= cus && 4 * outputs >= 3 * (int64_t)cus * 160 * WB_N) {
-        *mi = 5;
-        return n_out;
-    }
-    return 0;
+    if (((uintptr_t)W & 3u) != 0 || ((uintptr_t)Xq & 3u) != 0) return 0;
+    if (!force) return wide_rows(n_out, n_tok, nb, cus, mi);
+    *mi = pq2host::knob(pq2host::K_GEMM_WIDE_MI, 8) == 5 ? 5 : 8;
+    return wide_fits(n_out, n_tok, nb) ? n_out : 0;
 }
 
 // The wide kernel (mi = 8 or 5) over rows [0, n_out) of W / Y (the caller

@@ -5,6 +5,8 @@
 
 #include <stdint.h>
 
+#include <initializer_list>
+
 namespace pq2 {
 
 // RMSNorm -> FWHT -> Q8_1 of n_tok rows of nhb blocks of 1024: a workgroup per
@@ -88,6 +90,102 @@ inline int mid_pick(int64_t n_out, int64_t n_tok, int nb, int cus, float * us) {
         if (pick < 0 || t < *us) *us = t, pick = k;
     }
     return pick;
+}
+
+// ---- more than 16 tokens ---------------------------------------------------
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// What the wide kernel (gemm_wide.hip) needs of the sizes: whole pairs of blocks,
+// and buffer ranges that are ints
+inline bool wide_fits(int64_t n_out, int64_t n_tok, int nb) {
+    return nb >= 2 && nb % 2 == 0 && (uint64_t)n_out * 34 * (uint64_t)nb < (1ull << 31) &&
+           (uint64_t)n_tok * 36 * 4 * (uint64_t)nb < (1ull << 31);
+}
+
+// Rows [0, rows) of the product that the wide kernel takes, and its tile
+// height (*mi = 8: 256 rows, 5: 160 rows): the whole 256-row tiles whose
+// 256 x 256 tiles fill whole rounds of the device's CUs (the caller runs the
+// remaining rows on the 128-row kernel), or, short of one round, every row on
+// 256- or 160-row tiles where one round of them holds at least 3/4 of a full
+// round's outputs; 0 where the kernel's requirements do not hold or its tiles
+// would fill too little of a round.
+inline int64_t wide_rows(int64_t n_out, int64_t n_tok, int nb, int cus, int * mi) {
+    *mi = 8;
+    if (!wide_fits(n_out, n_tok, nb)) return 0;
+    const int64_t T = ceil_div(n_tok, 256);
+    if (4 * n_tok < 3 * T * 256) return 0;                                        // token tiles mostly empty
+    // 256-row tiles over the rows whose tiles fill whole rounds
+    const int64_t R = n_out / 256, rounds = R * T / cus;
+    if (rounds >= 1) return (rounds * cus / T < R ? rounds * cus / T : R) * 256;
+    // Less than one round: a round of wide tiles takes about the same time
+    // however many CUs it fills, so one pays where at least 3/4 of a full
+    // round's outputs are real (measured on MI355X, one process, us, LDS kernel
+    // -> wide: 17408x5120 M = 768 225 -> 181 (256 rows), M = 512 165 -> 138
+    // (160 rows), 6144x5120 M = 2048 191 -> 183 (256 rows); at 5/8 and below
+    // the LDS kernel stays faster: 17408x5120 M = 384 116 against 137,
+    // 5120x6144 M = 1024 126 against 160)
+    const int64_t outputs = n_out * n_tok;
+    if (ceil_div(n_out, 256) * T <= cus && 4 * outputs >= 3 * (int64_t)cus * 256 * 256) return n_out;
+    if (ceil_div(n_out, 160) * T <= cus && 4 * outputs >= 3 * (int64_t)cus * 160 * 256) {
+        *mi = 5;
+        return n_out;
+    }
+    return 0;
+}
+
+// Time (us) of tokens [0, cols) on the large tiles, rows as wide_rows gives
+// them: rounds of workgroups times what a round takes a block of K (MI355X: 4.5
+// us on 256-row tiles, 3.45 on 160-row ones, 1.42 on 128 x 128, 1.05 on 128 x 64;
+// 128 x 128 tiles that fill three rounds or more exactly take 1.55 to 1.6 each, so
+// that three do not pass for faster than one of 256-row tiles: 6144x5120 with 2048
+// tokens 187 us against 179, 12288x5120 with 1024 187 against 178)
+inline float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows, int mi) {
+    float us = 0.0f;
+    if (rows > 0) us = (mi == 8 ? 4.5f : 3.45f) * (float)ceil_div(ceil_div(rows, 32 * mi) * ceil_div(cols, 256), cus);
+    if (rows < n_out) {
+        // gemm_prefill_f16's choice
+        const int64_t R = ceil_div(n_out - rows, 128), T = ceil_div(cols, 128);
+        const int64_t full = R * T / cus, rest = R * T - full * cus;
+        if (2 * R * T <= cus) us += 1.05f;
+        else if (full >= 1 && rest > 0 && 2 * rest <= cus && full * cus % T == 0 &&
+                 (R - full * cus / T) * ceil_div(cols, 64) <= cus)
+            us += 1.42f * (float)full + 1.05f;
+        else us += (rest == 0 && full >= 3 ? 1.55f : 1.42f) * (float)ceil_div(R * T, cus);
+    }
+    return us * (float)nb;
+}
+
+// The tiles of a prefill: tokens [0, cols) on the large ones, the first rows of
+// them on the wide kernel (tile height mi), tokens [cols, n_tok) on the small
+// ones (gemm_mid.hip; cols = 0: all of them).  wide, small: the pointers let
+// these kernels run (and, for the small one, the sizes).  rows and mi come as
+// wide_rows gives them for every token; another plan has to be 5 % faster by its
+// estimate.  Small tiles take over the whole product where large ones would leave
+// most CUs idle, or the tokens past the whole large tiles where these would start
+// another round, and rows whose wide tiles are short of a round take 128-row
+// tiles where those have fewer empty tokens.  Measured (us, large tiles as
+// wide_rows has them -> this plan): 17408x5120 with 20 tokens 57 -> 17, 33 54 ->
+// 22, 100 57 -> 48, 140 101 -> 63, 400 159 -> 126; 5120x17408 with 100 132 -> 45, 800
+// 361 -> 213; 10240x5120 with 386 102 -> 69, 777 139 -> 129 (768 + 9 tokens), 1166 229 ->
+// 180; unchanged 17408x5120 with 1500, 10240x5120 with 1900.
+inline void prefill_plan(bool wide, bool small, int64_t n_out, int64_t n_tok, int nb, int cus, int64_t * cols,
+                         int64_t * rows, int * mi) {
+    float best = 0.95f * large_us(n_out, n_tok, nb, cus, *rows, *mi);
+    float us = 0.0f;
+    if (small) mid_pick(n_out, n_tok, nb, cus, &us);
+    if (small && us < best) best = us, *cols = 0, *rows = 0;
+    // wide_rows looks at the tokens that it is given only
+    if ((uint64_t)n_tok * 36 * 4 * (uint64_t)nb >= (1ull << 31)) return;
+    for (int64_t c : {n_tok, n_tok / 128 * 128, n_tok / 256 * 256}) {
+        if (c == 0 || (c < n_tok && !small)) continue;
+        us = 0.0f;
+        if (c < n_tok) mid_pick(n_out, n_tok - c, nb, cus, &us);
+        int m = 8;
+        const int64_t r = wide ? wide_rows(n_out, c, nb, cus, &m) : 0;
+        const float with = us + large_us(n_out, c, nb, cus, r, m), plain = us + large_us(n_out, c, nb, cus, 0, 8);
+        if (r > 0 && (c == n_tok || c % 256 == 0) && with < best) best = with, *cols = c, *rows = r, *mi = m;
+        if (plain < best) best = plain, *cols = c, *rows = 0;
+    }
 }
 
 }  // namespace pq2

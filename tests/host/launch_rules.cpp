@@ -17,4 +17,11 @@ float mid_us(int64_t n_out, int64_t n_tok, int nb, int cus) {
     pq2::mid_pick(n_out, n_tok, nb, cus, &us);
     return us;
 }
+void prefill_plan(int wide, int small, int64_t n_out, int64_t n_tok, int nb, int cus, int64_t * plan) {
+    int mi = 8;
+    plan[0] = n_tok;
+    plan[1] = wide ? pq2::wide_rows(n_out, n_tok, nb, cus, &mi) : 0;
+    pq2::prefill_plan(wide != 0, small != 0, n_out, n_tok, nb, cus, &plan[0], &plan[1], &mi);
+    plan[2] = plan[1] > 0 ? 32 * mi : 0;
+}
 }

@@ -51,3 +51,46 @@ def test_small_tile_shape(rules, n_out, n_in, n_tok, bm, bn, us):
     assert rules.mid_pick(I64(n_out), I64(n_tok), n_in // 128, CUS) == 1000 * bm + bn
     rules.mid_us.restype = ctypes.c_float
     assert 0.75 * us < rules.mid_us(I64(n_out), I64(n_tok), n_in // 128, CUS) < 1.25 * us
+
+
+def plan(rules, n_out, n_in, n_tok, wide=1, small=1):
+    out = (ctypes.c_int64 * 3)()
+    rules.prefill_plan(wide, small, I64(n_out), I64(n_tok), n_in // 128, CUS, out)
+    return tuple(out)
+
+
+# tokens and rows of the large tiles, and the height of their wide tiles (0: all
+# on the 128-row kernel); the tokens past them are on the small tiles
+@pytest.mark.parametrize("n_out,n_in,n_tok,cols,rows,bm", [
+    # small tiles only
+    (17408, 5120, 17, 0, 0, 0), (17408, 5120, 33, 0, 0, 0), (17408, 5120, 100, 0, 0, 0), (5120, 17408, 100, 0, 0, 0),
+    (1024, 5120, 512, 0, 0, 0), (1000, 5120, 200, 0, 0, 0), (129, 1024, 130, 0, 0, 0),
+    # large tiles, and the tokens past them on small ones
+    (10240, 5120, 777, 768, 0, 0), (17408, 5120, 777, 768, 17408, 256), (17408, 5120, 400, 384, 0, 0),
+    (12288, 5120, 1300, 1280, 12288, 256), (17408, 5120, 2100, 2048, 16384, 256), (5120, 17408, 800, 768, 0, 0),
+    # 128-row tiles only
+    (17408, 5120, 384, 384, 0, 0), (17408, 5120, 300, 300, 0, 0), (10240, 5120, 768, 768, 0, 0),
+    (6144, 5120, 1280, 1280, 0, 0), (12288, 5120, 640, 640, 0, 0), (4096, 4096, 2048, 2048, 0, 0),
+    # wide tiles: whole rounds, one round of 256 or of 160 rows
+    (17408, 5120, 2048, 2048, 16384, 256), (17408, 5120, 768, 768, 17408, 256), (17408, 5120, 512, 512, 17408, 160),
+    (5120, 6144, 2048, 2048, 5120, 160),
+    # one round of 256-row tiles, not three full ones of 128 x 128
+    (6144, 5120, 2048, 2048, 6144, 256), (12288, 5120, 1024, 1024, 12288, 256), (12288, 4096, 1024, 1024, 12288, 256),
+    (8192, 2048, 1536, 1536, 8192, 256), (6144, 5120, 1950, 1950, 0, 0)])
+def test_prefill_plan(rules, n_out, n_in, n_tok, cols, rows, bm):
+    assert plan(rules, n_out, n_in, n_tok) == (cols, rows, bm)
+
+
+@pytest.mark.parametrize("n_tok", [17, 33, 100, 384, 512, 768, 777, 1300, 2048, 4096, 100000])
+@pytest.mark.parametrize("n_out,n_in", [(17408, 5120), (5120, 17408), (10240, 5120), (1024, 5120), (300, 3072), (77, 1024)])
+def test_prefill_plan_is_launchable(rules, n_out, n_in, n_tok):
+    """Token ranges and rows that the launches take: the large tiles' tokens are
+    all or whole tiles, the wide rows all or whole tiles, and a kernel that the
+    pointers rule out is not used."""
+    for wide in (0, 1):
+        for small in (0, 1):
+            cols, rows, bm = plan(rules, n_out, n_in, n_tok, wide, small)
+            assert 0 <= cols <= n_tok and (cols == n_tok or cols % (256 if rows else 128) == 0)
+            assert 0 <= rows <= n_out and (rows in (0, n_out) or rows % bm == 0) and (rows > 0) == (bm > 0)
+            assert wide or rows == 0
+            assert small or cols == n_tok
