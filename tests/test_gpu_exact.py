@@ -137,14 +137,18 @@ EXACT_CASES = [
     # 3..4 tokens without it: the 4x4x4 MFMA streaming kernel
     (17408, 5120, 4, {"BONSAI_GEMM_BD": "0"}, 0, 0),
     (6144, 5120, 3, {"BONSAI_GEMM_BD": "0"}, 0, 0),
-    # 5..16 tokens: the streamed 16x16x32 int8 MFMA kernel
+    # 9..16 tokens on a tall matrix: 80x16 f16-MFMA tiles
     (17408, 5120, 13, {}, 0, 0),
+    # 5..16 tokens: the streamed 16x16x32 int8 MFMA kernel
+    (17408, 5120, 13, {"BONSAI_GEMM_MID": "0"}, 0, 0),
     (5120, 17408, 16, {}, 0, 0),
     (300, 5120, 9, {"BONSAI_GEMM_SMALL_CFG": "3"}, 0, 0),
     # <= 16 tokens with an unaligned X: the skinny kernel
     (200, 5120, 6, {"BONSAI_GEMM_BD": "0"}, 0, 4),
-    # f16-MFMA prefill tile GEMM: 64- and 128-token tiles, ragged edges
+    # a few dozen tokens: small f16-MFMA tiles
     (1000, 5120, 17, {}, 0, 0),
+    # f16-MFMA prefill tile GEMM: 64- and 128-token tiles, ragged edges
+    (1000, 5120, 17, {"BONSAI_GEMM_WIDE": "0"}, 0, 0),
     (300, 6144, 77, {"BONSAI_GEMM_F16_BN": "128"}, 0, 0),
     (129, 1024, 130, {"BONSAI_GEMM_F16_BN": "64"}, 0, 0),
     (17408, 5120, 512, {}, 0, 0),

@@ -94,11 +94,12 @@ def test_graph_replays_of_gemv_gemm_and_fused_launches():
     replay_and_check(g, outs, refs, lambda: B.gemv(W, xq, other, n_out, n_in))
 
 
-@pytest.mark.parametrize("wide,n_out,n_tok", [("2", 600, 300), ("1", 17408, 1024)])
+@pytest.mark.parametrize("wide,n_out,n_tok", [("2", 600, 300), ("1", 17408, 1024), ("1", 17408, 1100)])
 def test_graph_replays_of_wide_prefill_gemm(wide, n_out, n_tok, knobs):
     """The wide prefill kernel in a graph: forced on a ragged shape, and by
     the default rule on a shape it splits into the wide launch and the
-    128-row launch for the remaining rows."""
+    128-row launch for the remaining rows, and on one whose last 76 tokens it
+    gives to small tiles."""
     knobs.set("BONSAI_GEMM_WIDE", wide)
     case(f"graph: prefill GEMM {n_out}x5120x{n_tok}, BONSAI_GEMM_WIDE={wide}")
     n_in = 5120

@@ -5,8 +5,8 @@ descriptor whose range is the matrix: they switch to 64-bit addresses and clamp 
 trailing unit's pieces to the end of W themselves.  The small-batch kernels
 for 3..16 tokens address W with unsigned 32-bit per-lane offsets, which must
 hold up to 4 GiB.  From 4 GiB on, those kernels are skipped and the others
-(per-token planes, 4x4x4 MFMA, the skinny kernel, the prefill tile GEMM) use
-64-bit offsets.
+(per-token planes, 4x4x4 MFMA, the skinny kernel, the small- and large-tile
+prefill GEMMs) use 64-bit offsets.
 
 The matrices are filled on the device (random code bytes, random finite fp16
 block scales), so only a row sample goes to the host: the first rows, rows on
@@ -134,12 +134,23 @@ def test_gemv_large_matrix(mats, key):
         check_gemv_rows(y, W, n_out, n_in, O.quantize_q8_1(x, True), 9804)
 
 
-@pytest.mark.parametrize("key,n_tok", [("2g_5120", t) for t in (2, 3, 4, 6, 8, 12, 64)] +
-                         [("4g_5120", t) for t in (2, 3, 8, 16, 40)] + [("2g_17408", 2), ("2g_17408", 8)])
-def test_gemm_large_matrix(mats, key, n_tok):
+# env: the small-tile GEMM, which takes these sizes from 9 tokens up, switched off,
+# so that the streamed kernel (12 tokens), the skinny kernel (16, past 4 GiB) and
+# the 128-row prefill kernel (40 and 64) run
+NO_SMALL_TILES = {"BONSAI_GEMM_MID": 0, "BONSAI_GEMM_WIDE": 0}
+
+
+@pytest.mark.parametrize("key,n_tok,env", [("2g_5120", t, {}) for t in (2, 3, 4, 6, 8, 12, 64)] +
+                         [("2g_5120", t, NO_SMALL_TILES) for t in (12, 64)] +
+                         [("4g_5120", t, {}) for t in (2, 3, 8, 16, 40)] +
+                         [("4g_5120", t, NO_SMALL_TILES) for t in (16, 40)] +
+                         [("2g_17408", 2, {}), ("2g_17408", 8, {})])
+def test_gemm_large_matrix(mats, key, n_tok, env, knobs):
     n_out, n_in = SHAPES[key]
     rs = 34 * (n_in // 128)
-    case(f"large GEMM {n_out}x{n_in} ({n_out * rs / GIB:.2f} GiB), {n_tok} tokens")
+    case(f"large GEMM {n_out}x{n_in} ({n_out * rs / GIB:.2f} GiB), {n_tok} tokens {env}")
+    for k, v in env.items():
+        knobs.set(k, v)
     W = mats(key)
     assert W.numel() == n_out * rs
     X = np.stack([O.fwht(O.gen_normal(9900 + t, n_in)) for t in range(n_tok)])

@@ -99,13 +99,16 @@ def test_mid_scales_at_the_ends(knobs):
     assert np.max(np.abs(got[fine] - ref[fine])) <= TOL * np.max(np.abs(ref[fine]))
 
 
-@pytest.mark.parametrize("n_out,n_in,n_tok", [(1024, 5120, 512), (5120, 17408, 100), (17408, 5120, 33), (17408, 5120, 12),
-                                              (6144, 5120, 651), (10240, 5120, 777), (17408, 5120, 400),
-                                              (17408, 5120, 2100)])
-def test_mid_default_dispatch(n_out, n_in, n_tok):
+# the last figure is the tokens that stay on the large tiles (or, up to 16, on the
+# streamed kernel)
+@pytest.mark.parametrize("n_out,n_in,n_tok,cols", [
+    (1024, 5120, 512, 0), (5120, 17408, 100, 0), (17408, 5120, 33, 0), (17408, 5120, 12, 0), (6144, 5120, 651, 640),
+    (10240, 5120, 777, 768), (17408, 5120, 400, 384), (17408, 5120, 2100, 2048)])
+def test_mid_default_dispatch(n_out, n_in, n_tok, cols, knobs):
     """Shapes the default rule gives to this kernel, whole or the tokens past the
     large tiles' whole ones, with and without a workspace (the same bytes), on a
-    row sample."""
+    row sample.  Without this kernel (BONSAI_GEMM_MID=0) the tokens before those
+    keep their bytes and the others, whose sums it adds in another order, do not."""
     case(f"mid GEMM by default: {n_out}x{n_in}x{n_tok}")
     W = O.gen_weights(6400 + n_out, n_out, n_in)
     X = O.gen_normal(6401 + n_tok, n_tok * n_in).reshape(n_tok, n_in)
@@ -121,6 +124,10 @@ def test_mid_default_dispatch(n_out, n_in, n_tok):
     Ws = np.concatenate([W[r * rb:(r + 1) * rb] for r in rows])
     assert np.all(np.isfinite(got))
     assert normwise(got[rows], O.gemm(Ws, Xq, rows.size, n_in, n_tok, nthreads=16)) <= TOL
+    knobs.set("BONSAI_GEMM_MID", 0)
+    without = gemm(Wd, Xd, n_out, n_in, n_tok)
+    np.testing.assert_array_equal(got[:, :cols].view(np.uint32), without[:, :cols].view(np.uint32))
+    assert np.all(np.any(got[:, cols:] != without[:, cols:], axis=0))
 
 
 def test_mid_stored_sum_up_to_16_tokens(knobs):

@@ -720,10 +720,14 @@ def test_gemv_shared_tail_fused_and_grouped(kind, knobs):
             assert normwise(got, O.gemv(W, xqh, n, n_in, nthreads=16)) <= TOL
 
 
-def test_gemm_subnormal_and_zero_block_scales():
-    """Blocks whose fp16 scale is subnormal or zero (the prefill kernel
-    multiplies the scale into its f16 operand)."""
-    case("gemm 200x2048x64 with subnormal / zero block scales")
+@pytest.mark.parametrize("wide", [None, 0])
+def test_gemm_subnormal_and_zero_block_scales(wide, knobs):
+    """Blocks whose fp16 scale is subnormal or zero, by default (small tiles) and
+    on the 128-row prefill kernel (BONSAI_GEMM_WIDE=0), which multiplies the
+    scale into its f16 operand."""
+    case(f"gemm 200x2048x64 with subnormal / zero block scales, BONSAI_GEMM_WIDE={wide}")
+    if wide is not None:
+        knobs.set("BONSAI_GEMM_WIDE", wide)
     n_out, n_in, n_tok = 200, 2048, 64
     W = O.gen_weights(1500, n_out, n_in).copy()
     nb = n_in // 128
