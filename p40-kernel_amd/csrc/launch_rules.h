@@ -136,9 +136,9 @@ inline int64_t wide_rows(int64_t n_out, int64_t n_tok, int nb, int cus, int * mi
 // Time (us) of tokens [0, cols) on the large tiles, rows as wide_rows gives
 // them: rounds of workgroups times what a round takes a block of K (MI355X: 4.5
 // us on 256-row tiles, 3.45 on 160-row ones, 1.42 on 128 x 128, 1.05 on 128 x 64;
-// 128 x 128 tiles that fill three rounds or more exactly take 1.55 to 1.6 each, so
-// that three do not pass for faster than one of 256-row tiles: 6144x5120 with 2048
-// tokens 187 us against 179, 12288x5120 with 1024 187 against 178)
+// a product that fills three rounds of 128 x 128 or more exactly takes 1.55 to 1.6
+// each, so that three do not pass for faster than one of 256-row tiles: 12288x5120
+// with 1024 tokens 184 us against 177, 8192x2048 with 1536 82 against 78)
 inline float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows, int mi) {
     float us = 0.0f;
     if (rows > 0) us = (mi == 8 ? 4.5f : 3.45f) * (float)ceil_div(ceil_div(rows, 32 * mi) * ceil_div(cols, 256), cus);
@@ -150,7 +150,7 @@ inline float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows
         else if (full >= 1 && rest > 0 && 2 * rest <= cus && full * cus % T == 0 &&
                  (R - full * cus / T) * ceil_div(cols, 64) <= cus)
             us += 1.42f * (float)full + 1.05f;
-        else us += (rest == 0 && full >= 3 ? 1.55f : 1.42f) * (float)ceil_div(R * T, cus);
+        else us += (rows == 0 && rest == 0 && full >= 3 ? 1.55f : 1.42f) * (float)ceil_div(R * T, cus);
     }
     return us * (float)nb;
 }

@@ -76,7 +76,9 @@ def plan(rules, n_out, n_in, n_tok, wide=1, small=1):
     (5120, 6144, 2048, 2048, 5120, 160),
     # one round of 256-row tiles, not three full ones of 128 x 128
     (6144, 5120, 2048, 2048, 6144, 256), (12288, 5120, 1024, 1024, 12288, 256), (12288, 4096, 1024, 1024, 12288, 256),
-    (8192, 2048, 1536, 1536, 8192, 256), (6144, 5120, 1950, 1950, 0, 0)])
+    (8192, 2048, 1536, 1536, 8192, 256), (6144, 5120, 1950, 1950, 0, 0),
+    # 256-row tiles and three full rounds of 128 x 128 for the rows past them
+    (28672, 8192, 1061, 1024, 16384, 256)])
 def test_prefill_plan(rules, n_out, n_in, n_tok, cols, rows, bm):
     assert plan(rules, n_out, n_in, n_tok) == (cols, rows, bm)
 
