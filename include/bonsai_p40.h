@@ -64,18 +64,28 @@ int bonsai_p40_quant_activations(const float * x, void * out, int64_t n, bonsai_
 // per-token activation planes; 3..8 the block-diagonal 16x16x64 int8 MFMA
 // kernel, except 4 tokens on 1024-, 5120- and 6144-column rows and 3 on
 // 1024- and 6144-column rows, which take the 4x4x4 int8 MFMA streaming
-// kernel; 9..16 the streamed 16x16x32 int8 MFMA kernel, or on tall matrices
-// (17408 rows) f16-MFMA 80x16 tiles that read s as it does; larger n_tok the
-// f16-MFMA tile GEMMs: small tiles with K split over a workgroup's waves
-// where larger ones would leave CUs idle, for all tokens or those past the
-// whole larger tiles (n_in % 1024 == 0, 16-byte aligned W), else 128- to
-// 256-row tiles (other alignments: 64-bit-offset MFMA kernels).  The GEMV and the streamed small-batch kernels subtract each Q8_1
-// block's stored sum s as the reference does (src/pq2_0.h:169); the tile GEMMs
-// and the kernels for other alignments multiply (code - 1) by q directly and
-// do not read s.  The two agree for blocks whose s is the sum of their q, which
-// holds for every block this library's or the reference's quantiser writes.  Errors: 1 if n_in <= 0 or n_in % 128 != 0, Xq is not 4-byte or W
-// not 2-byte aligned, or n_out, n_tok or n_in / 128 is too large for the
-// launch; 0 (no-op) if n_out <= 0 or n_tok <= 0.
+// kernel; 9..16 the streamed 16x16x32 int8 MFMA kernel, or f16-MFMA 80x16
+// tiles that read s as it does on matrices of more than 64 rows a CU where
+// rounds of 80 rows a CU, rounded up, are no more than n_out in rounds of 64
+// (n_in % 1024 == 0, n_in >= 5120, 16-byte aligned W); larger n_tok the
+// f16-MFMA tile GEMMs: small tiles with K split over a workgroup's waves where
+// larger ones would leave CUs idle, for all tokens or those past the whole
+// larger tiles (n_in % 1024 == 0, 16-byte aligned W), else 128- to 256-row
+// tiles (other alignments: 64-bit-offset MFMA kernels).  The GEMV, the streamed small-batch kernels and the 80x16 tiles
+// subtract each Q8_1 block's stored sum s as the reference does
+// (src/pq2_0.h:169); the GEMMs for more than 16 tokens and the kernels for
+// other alignments multiply (code - 1) by q directly and do not read s.  The
+// two agree for blocks whose s is the sum of their q, which holds for every
+// block this library's or the reference's quantiser writes.
+// The kernels add in different orders, each within fp32 rounding of the sum:
+// the last bits of a token's column may depend on n_tok, on the token's place
+// in the call and on n_out (so on how a prompt is chunked or a matrix sharded
+// by rows); the same call gives the same bytes every time.  A block scale that
+// is infinite gives infinities and NaN, and which of them depends on the
+// kernel.
+// Errors: 1 if n_in <= 0 or n_in % 128 != 0, Xq is not 4-byte or W not 2-byte
+// aligned, or n_out, n_tok or n_in / 128 is too large for the launch; 0
+// (no-op) if n_out <= 0 or n_tok <= 0.
 int bonsai_p40_gemm(const void * W, const void * Xq, float * Y,
                     int64_t n_out, int64_t n_in, int64_t n_tok, bonsai_stream stream);
 

@@ -104,10 +104,10 @@ quant_kernel(const float * __restrict__ x, uint8_t * __restrict__ q, int nchunk,
 // the pre-pass.  Output chunk-major (block (c, t) at c * n_tok + t).
 // Workgroups go to the 8 XCDs in turn: each XCD takes a contiguous run of
 // tokens, whose 36-byte blocks share lines of its L2.  VALU-bound (~600
-// instructions a block) at about the time its bytes take: with the row read
-// once and the tokens dealt by XCD 2048 x 5120 went 20.1 -> 17.0 us (54 MB,
-// 3.2 TB/s), 2048 x 17408 67.6 -> 52.6.  Collecting 2 or 4 tokens a workgroup
-// to write longer runs measured slower (18.5, 22.1).
+// instructions a block) at 1.5 times what its bytes take: with the row read
+// once and the tokens dealt by XCD 2048 x 5120 went 18.9 -> 15.9 us (54 MB,
+// 3.4 TB/s), 2048 x 17408 72 -> 55.  Collecting 2 or 4 tokens a workgroup to
+// write longer runs measured slower (18.5, 22.1).
 template <bool VEC, bool SIGNS, int KEEP>
 __global__ void __launch_bounds__(1024)
 rms_rot_quant_kernel(const float * __restrict__ x, const float * __restrict__ w,
