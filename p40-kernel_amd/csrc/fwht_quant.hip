@@ -330,7 +330,10 @@ int bonsai_p40_rmsnorm_fwht_quant(const float * x, const float * w, const float 
     const int nw = keep == 1 ? nhb : keep == 2 ? (nhb + 1) / 2 : 16;
     const bool vec = al16(x) && al16(w) && al16(signs);
     hipStream_t st = (hipStream_t)stream;
-    const bool per_block = pq2::rms_per_block(n_tok, nhb, pq2host::device_info().cus);
+    // (CUs of the first device used: they move a line between kernels that write
+    // the same bytes, and asking for the current device costs 0.07 us a call)
+    static const int cus = pq2host::device_info().cus;
+    const bool per_block = pq2::rms_per_block(n_tok, nhb, cus);
 #define PQ2_RMS_LAUNCH(V, S)                                                                        \
     if (per_block)                                                                                  \
         hipLaunchKernelGGL((rms_rot_quant_block_kernel<V, S>), dim3((unsigned)(n / HBLK), (unsigned)n_tok), \

@@ -167,7 +167,9 @@ inline float large_us(int64_t n_out, int64_t cols, int nb, int cus, int64_t rows
 // wide_rows has them -> this plan): 17408x5120 with 20 tokens 57 -> 17, 33 54 ->
 // 22, 100 57 -> 48, 140 101 -> 63, 400 159 -> 126; 5120x17408 with 100 132 -> 45, 800
 // 361 -> 213; 10240x5120 with 386 102 -> 69, 777 139 -> 129 (768 + 9 tokens), 1166 229 ->
-// 180; unchanged 17408x5120 with 1500, 10240x5120 with 1900.
+// 180; unchanged 17408x5120 with 1500, 10240x5120 with 1900.  Not a matter of the
+// workspace, with which wide tiles are up to 5 % faster: the bytes have to be the
+// same with and without one (8704x5120 with 960 tokens and a workspace pays 3 %).
 inline void prefill_plan(bool wide, bool small, int64_t n_out, int64_t n_tok, int nb, int cus, int64_t * cols,
                          int64_t * rows, int * mi) {
     float best = 0.95f * large_us(n_out, n_tok, nb, cus, *rows, *mi);
