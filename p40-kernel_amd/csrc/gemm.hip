@@ -1327,7 +1327,8 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
     // 32-bit per-lane offsets: a matrix of 4 GiB or more takes the kernels
     // below them, which use 64-bit offsets
     const bool off32 = (uint64_t)n_out * PQ2_BYTES * (uint64_t)nb < (1ull << 32);
-    const int bd_cfg = knob(pq2host::K_GEMM_BD, -1) < 0 ? bd_choice(nb, n_out, n_tok, gemm_cu_count())
+    const int cus = gemm_cu_count();                            // one look-up a call (0.07 us)
+    const int bd_cfg = knob(pq2host::K_GEMM_BD, -1) < 0 ? bd_choice(nb, n_out, n_tok, cus)
                                                               : knob(pq2host::K_GEMM_BD, 0);
     if (off32 && bd_cfg > 0 && n_tok >= 3 && n_tok <= 8 && nb % 2 == 0 && nb >= 16 && ((uintptr_t)W & 3u) == 0 &&
         ((uintptr_t)Xq & 15u) == 0) {
@@ -1345,7 +1346,7 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
     }
     // tall matrices at 9 to 16 tokens (its own rule; the small kernels' knobs keep theirs)
     if (n_tok >= 9 && n_tok <= 16 && knob(pq2host::K_GEMM_SMALL, 0) == 0 && knob(pq2host::K_GEMM_SMALL_CFG, 0) == 0) {
-        const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, gemm_cu_count(), st);
+        const int rc = pq2::gemm_mid(W, Xq, Y, n_out, n_tok, nb, cus, st);
         if (rc >= 0) return rc;
     }
     const size_t skinny_lds = (size_t)4 * 16 * PQ2_BYTES * (nb / 4) + 4096;
@@ -1374,7 +1375,7 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
         // measured on MI355X: 16-row workgroups, K split 8 ways up to 8 tokens
         // (more waves in flight); past that see the rule
         if (n_tok <= 8 && nb >= 16) return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
-        const pq2::SmallShape shape = pq2::small_shape(n_out, nb, gemm_cu_count());
+        const pq2::SmallShape shape = pq2::small_shape(n_out, nb, cus);
         if (shape.rt == 2) return launch_small_nt<2, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
         if (shape.ks == 8) return launch_small_nt<1, 8>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
         return launch_small_nt<1, 4>(w, x, Y, (int)n_out, (int)n_tok, nb, st);
@@ -1388,7 +1389,6 @@ int gemm_dispatch(const void * W, const void * Xq, float * Y, int64_t n_out, int
         // long prompts: the 256-row wide kernel (gemm_wide.hip) over the rows
         // whose tiles fill whole rounds of CUs, the 128-row kernel for the rest
         const int wide = n_tok > 16 ? knob(pq2host::K_GEMM_WIDE, 1) : 0;
-        const int cus = gemm_cu_count();
         int mi = 8;
         int64_t cols = n_tok;                                   // tokens of the large tiles; the rest on small ones
         int64_t rows = wide != 0 ? pq2::gemm_wide_rows(W, Xq, n_out, n_tok, nb, cus, wide == 2, &mi) : 0;
